@@ -184,12 +184,31 @@ def _splits12(splits):
     return sp + (None,) * (12 - len(sp))
 
 
+# A block's convolution pair runs in the few-row kernels (csrc/gemm_short.hip, three launches each
+# way) up to this many floating-point operations in its forward products, and up to this many
+# edges; above either the tiled GEMMs fill the chip.  Measured, us forward + backward (captured,
+# few-row / tiled): C = 128 lmax 2 (2.75 MFLOP an edge) 282 / 354 at 6,000 edges, 549 / 459 at
+# 12,000; C = 128 lmax 4 (11.1) 327 / 554 at 1,620, 543 / 555 at 3,000; C = 64 lmax 2 (0.69) 194 /
+# 255 at 12,000, 303 / 291 at 20,000.
+SHORT_PAIR_MAX_FLOPS = 2.2e10
+SHORT_PAIR_MAX_EDGES = 16384
+
+
+def _short_pair(E: int, C: int, L: int, sp: tuple, *biases) -> bool:
+    """Whether the few-row kernels take a pair of E edges: split-fp16 mode, every weight pre-split
+    and both m = 0 biases present."""
+    mac = 2 * ((2 * L + 1) * 2 * (L + 1) + (L + 1) ** 2) + 18 * (L * L + (L - 1) ** 2)   # flops / C^2
+    return (0 < E <= min(SHORT_PAIR_MAX_EDGES, SHORT_PAIR_MAX_FLOPS / (mac * C * C)) and C <= 256
+            and all(t is not None for t in sp + biases) and _lib.get_matmul_mode() == _lib.MATMUL_SPLIT_F16)
+
+
 def conv_pair_fwd(X: list, conv1, conv2, C: int, splits, m0=None):
     """conv1 + gate + conv2 of one block on X = [X_m0, X_m1, X_m2].  Each entry of X is set
     to None once its GEMM has read it, so a caller that hands over its only references
     frees the (E, 18C) gather output while the block runs.  m0: None, or conv1 m = 0's
     (Y0, Z0) computed already (X_m0 is then None).  Returns (Zo0, Zo1, Zo2) and the
-    pre-activations (Y0, Y1, Y2) the backward needs.
+    pre-activations (Y0, Y1, Y2) the backward needs.  On few edges (_short_pair) one call of
+    fu_so2_pair_fwd does all of it.
 
     After conv1 m = 0 (whose gate columns the complex gate epilogues read), conv1 m = 1 and
     conv2 m = 1 run on the current stream while conv1 m = 2, conv2 m = 2 and conv2 m = 0 run
@@ -200,6 +219,17 @@ def conv_pair_fwd(X: list, conv1, conv2, C: int, splits, m0=None):
     dev = X[1].device
     L = _degrees(W0, C)
     sp = _splits12(splits)
+    if m0 is None and _short_pair(X[1].shape[0], C, L, sp, b0, c0):
+        X0, X1, X2 = (_lib.require(x, torch.float32, "X_m") for x in X)
+        X[0] = X[1] = X[2] = None
+        E = X1.shape[0]
+        f = lambda n: torch.empty(E, n, device=dev, dtype=torch.float32)
+        Y, Z, Zo = ([f(n * C) for n in ns] for ns in
+                    ((2 * L + 1, 2 * L, 2 * L - 2), (L + 1, 2 * L, 2 * L - 2), (L + 1, 2 * L, 2 * L - 2)))
+        _lib.call("fu_so2_pair_fwd", X0.data_ptr(), X1.data_ptr(), X2.data_ptr(), sp[8].data_ptr(), b0.data_ptr(),
+                  sp[0].data_ptr(), sp[2].data_ptr(), sp[10].data_ptr(), c0.data_ptr(), sp[4].data_ptr(),
+                  sp[6].data_ptr(), *(t.data_ptr() for t in (*Y, *Z, *Zo)), E, C, L, _lib.stream_ptr(dev))
+        return tuple(Zo), tuple(Y)
     if m0 is None:
         Y0, Z0 = _conv1_gate_m0(_lib.require(X[0], torch.float32, "X_m0"), W0, b0, C, L, _lib.stream_ptr(dev),
                                 sp[8])
@@ -249,6 +279,11 @@ def conv_pair_bwd(Y, conv1, conv2, C: int, splits, g: list):
     g1 = torch.zeros(E, 2 * L * C, device=dev) if g[1] is None else g[1].contiguous()
     g2 = torch.zeros(E, 2 * (L - 1) * C, device=dev) if g[2] is None else g[2].contiguous()
     g[0] = g[1] = g[2] = None
+    if _short_pair(E, C, L, sp):
+        outs = [f(E, n * C) for n in (2 * L + 1, 2 * L, 2 * L - 2, L, L - 1, 2 * L + 2, 4 * L, 4 * L - 4)]
+        _lib.call("fu_so2_pair_bwd", *(t.data_ptr() for t in (g0, g1, g2, Y0, Y1, Y2, sp[9], sp[1], sp[3], sp[11],
+                                                              sp[5], sp[7], *outs)), E, C, L, st)
+        return tuple(outs[5:])
     gy1, ps1 = f(E, 2 * R1t.shape[0]), f(E, R1t.shape[0])
     gy2, ps2 = f(E, 2 * R2t.shape[0]), f(E, R2t.shape[0])
     side = _lib.side_stream(dev)

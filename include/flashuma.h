@@ -356,6 +356,26 @@ int fu_linear_weight_split(const float* W, int64_t ldw, int32_t N, int32_t K, vo
 int fu_linear_resident(const float* A, int64_t lda, const void* W2, const float* bias, float* Y, int64_t ldy,
                        int64_t M, int32_t N, int32_t K, void* stream);
 
+/* The SO(2) convolution pair of a block on few edges (model.py:150-154), split-fp16 mode only
+ * (FU_ERR_UNSUPPORTED otherwise): conv1 + gate + conv2 in three launches, and their input
+ * gradients in three, each 32 x 64 output tile's K range split over the waves of a workgroup.  The
+ * arrays are contiguous: X_m / gX_m (E, 2 (lmax + 1) C | 4 lmax C | 4 (lmax - 1) C), Y_m / gY_m
+ * (E, (2 lmax + 1) C | 2 lmax C | 2 (lmax - 1) C), Z_m, O_m and G_m (E, (lmax + 1) C | 2 lmax C |
+ * 2 (lmax - 1) C), in the layouts of fu_linear_gate and fu_complex_linear_gate.  Weights pre-split:
+ * W0 / V0 (conv1 / conv2, m = 0, biases b0, c0; W0's rows gate-paired) by fu_linear_weight_split, W1,
+ * W2, V1, V2 (m = 1, 2) by fu_complex_weight_split; the *t ones are those of the input gradients
+ * (transposed, complex conjugated).  The backward's P1 (E, lmax C) and P2 (E, (lmax - 1) C) are
+ * workspaces.  Results as the tiled entry points' up to the order of the fp32 sums.  All pointers
+ * 16-byte aligned; C a multiple of 64 up to 256, lmax 2 to 4, 0 <= E <= 2^24. */
+int fu_so2_pair_fwd(const float* X0, const float* X1, const float* X2, const void* W0, const float* b0,
+                    const void* W1, const void* W2, const void* V0, const float* c0, const void* V1, const void* V2,
+                    float* Y0, float* Y1, float* Y2, float* Z0, float* Z1, float* Z2, float* O0, float* O1, float* O2,
+                    int64_t E, int32_t C, int32_t lmax, void* stream);
+int fu_so2_pair_bwd(const float* G0, const float* G1, const float* G2, const float* Y0, const float* Y1,
+                    const float* Y2, const void* W0t, const void* W1t, const void* W2t, const void* V0t,
+                    const void* V1t, const void* V2t, float* gY0, float* gY1, float* gY2, float* P1, float* P2,
+                    float* gX0, float* gX1, float* gX2, int64_t E, int32_t C, int32_t lmax, void* stream);
+
 /* The radial output layer fused with the gather-rotate forward (lmax 2, C = 128; replaces
  * model.py:149 rad_out = h2 W_rad1_3^T + b_rad1_3 followed by ops/gather.py:34-154
  * gather_wigner_split, whose only reader of rad_out in the forward is the gather): writes rad

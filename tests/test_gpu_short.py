@@ -1,0 +1,95 @@
+"""The few-row kernels of the SO(2) convolution pair (fu_so2_pair_fwd / _bwd) against float64, at the
+edges of their 32-row tiles, for every lmax and several widths (K ranges that do not divide evenly
+over the waves), and where the fp16 window rule sends a segment to the two-loop products."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(cuda, M, C, L, ramp=0.0):
+    """A pair on the GPU; with ramp > 0 the operands' columns carry 2^t and the weights' 2^-t, t
+    ramping over [-ramp, ramp] along K: the same products, opposite magnitudes."""
+    from ops import gating
+    from ops.linear import complex_weight_split, linear_weight_split
+    g = torch.Generator().manual_seed(M + 7 * C + L)
+    r = lambda *s: torch.randn(*s, generator=g)
+    n0, n1, n2 = (L + 1) * C, L * C, (L - 1) * C
+    t = lambda K: torch.exp2(torch.round(torch.linspace(-ramp, ramp, K)))
+    w = lambda n, k: r(n, k) / k ** 0.5
+    X = [r(M, 2 * n0), r(M, 4 * n1), r(M, 4 * n2)]
+    W0, b0, V0, c0 = w((2 * L + 1) * C, 2 * n0), r((2 * L + 1) * C) * 0.3, w(n0, n0), r(n0) * 0.3
+    R1, I1, R2, I2 = w(n1, 2 * n1), w(n1, 2 * n1), w(n2, 2 * n2), w(n2, 2 * n2)
+    S1, T1, S2, T2 = w(n1, n1), w(n1, n1), w(n2, n2), w(n2, n2)
+    f0, f1, f2 = t(2 * n0), t(2 * n1), t(2 * n2)
+    Xs = [X[0] * f0, X[1] * torch.cat([f1, f1]), X[2] * torch.cat([f2, f2])]
+    rows = gating.gate_paired_rows(C, L)
+    d = lambda a: a.contiguous().to(cuda)
+    A0, P1, Q1, P2, Q2 = W0[rows] / f0, R1 / f1, I1 / f1, R2 / f2, I2 / f2
+    conv1 = [d(A0), d(b0[rows]), d(A0.t()), d(P1), d(Q1), d(P1.t()), d(-Q1.t()), d(P2), d(Q2), d(P2.t()), d(-Q2.t())]
+    conv2 = [d(V0), d(c0), d(V0.t()), d(S1), d(T1), d(S1.t()), d(-T1.t()), d(S2), d(T2), d(S2.t()), d(-T2.t())]
+    cw = [conv1[3:5], conv1[5:7], conv1[7:9], conv1[9:11], conv2[3:5], conv2[5:7], conv2[7:9], conv2[9:11]]
+    sp = tuple(complex_weight_split(*p) for p in cw) + tuple(
+        linear_weight_split(v) for v in (conv1[0], conv1[2], conv2[0], conv2[2]))
+    cot = [r(M, n0), r(M, 2 * n1), r(M, 2 * n2)]
+    from oracle import ops_ref as R
+
+    def ref_fn(x0, x1, x2):
+        y = (x0 @ W0.double().T + b0.double(), x1 @ R.pack_so2(R1.double(), I1.double()).T,
+             x2 @ R.pack_so2(R2.double(), I2.double()).T)
+        z0, z1, z2 = R.gating(*y, C) if L == 2 else R.gating_lmax(*y, C, L)
+        return (z0 @ V0.double().T + c0.double(), z1 @ R.pack_so2(S1.double(), T1.double()).T,
+                z2 @ R.pack_so2(S2.double(), T2.double()).T)
+
+    Xd = [x.double().requires_grad_() for x in X]
+    ref = ref_fn(*Xd)
+    gref = torch.autograd.grad(ref, Xd, [c.double() for c in cot])
+    scale = [f0, torch.cat([f1, f1]), torch.cat([f2, f2])]
+    gref = [a / s.double() for a, s in zip(gref, scale)]
+    return [x.to(cuda) for x in Xs], conv1, conv2, sp, [c.to(cuda) for c in cot], list(ref) + gref
+
+
+def _run(X, conv1, conv2, C, sp, cot):
+    from ops import gating
+    Xg = [x.clone().requires_grad_() for x in X]
+    z = gating.conv1_gate_conv2(*Xg, conv1, conv2, C, sp)
+    return [t.detach() for t in z] + list(torch.autograd.grad(z, Xg, cot))
+
+
+def _err(got, ref):
+    return [((a.double().cpu() - b.detach()).norm() / b.detach().norm()).item() for a, b in zip(got, ref)]
+
+
+@pytest.mark.parametrize("M,C,L,ramp", [
+    (1, 128, 2, 0), (32, 128, 2, 0), (33, 128, 2, 0), (300, 128, 2, 0), (77, 64, 2, 0), (40, 256, 2, 0), (65, 64, 3, 0),
+    (100, 128, 3, 0), (150, 64, 4, 0), (95, 128, 4, 0), (70, 128, 2, 4), (70, 128, 2, 12), (70, 64, 4, 12)])
+def test_short_pair(cuda, monkeypatch, M, C, L, ramp):
+    """Outputs and input gradients, normwise: two products in a row of 22-bit operands and fp32 sums
+    (each at most 2^-21 relative, measured 2-4e-7) and no worse than 1.5x the tiled kernels' error;
+    twice the same bits."""
+    from ops import _lib, gating
+    X, conv1, conv2, sp, cot, ref = _pair(cuda, M, C, L, ramp)
+    calls = []
+    real = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    got = _run(X, conv1, conv2, C, sp, cot)
+    assert calls == ["fu_so2_pair_fwd", "fu_so2_pair_bwd"]
+    again = _run(X, conv1, conv2, C, sp, cot)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    monkeypatch.setattr(gating, "SHORT_PAIR_MAX_EDGES", 0)
+    tiled = _run(X, conv1, conv2, C, sp, cot)
+    for e, t in zip(_err(got, ref), _err(tiled, ref)):
+        assert e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
+
+
+def test_short_pair_nonfinite_rows_stay_apart(cuda):
+    """An infinite and a NaN element make their own rows non-finite and leave the others' bits."""
+    X, conv1, conv2, sp, cot, _ = _pair(cuda, 64, 128, 2)
+    clean = _run(X, conv1, conv2, 128, sp, cot)
+    X[0][3, 40], X[1][50, 7] = float("inf"), float("nan")
+    got = _run(X, conv1, conv2, 128, sp, cot)
+    ok = torch.ones(64, dtype=torch.bool, device=cuda)
+    ok[3] = ok[50] = False
+    for a, b in zip(got, clean):
+        assert torch.equal(a[ok], b[ok])
+    assert not torch.isfinite(got[0][3]).all() and not torch.isfinite(got[1][50]).all()
