@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256, 2) void linear_resident_kernel(const float* __
   const int nb = (N + 31) / 32;
   const int ntiles = (N + 127) / 128;
   const uint4* wf = W2 + lane;
-  for (int nt = 0; nt < ntiles; ++nt) {
+  for (int nt = (int)blockIdx.y; nt < ntiles; nt += (int)gridDim.y) {
     int cb[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -220,7 +220,13 @@ extern "C" int fu_linear_resident(const float* A, int64_t lda, const void* W2, c
   const uint4* w2 = static_cast<const uint4*>(W2);
   const float* cinv = reinterpret_cast<const float*>(w2 + resident_frag_vectors(N, K));
   const int* summary = reinterpret_cast<const int*>(cinv + resident_cols(N)) + resident_cols(N);
-  const dim3 grid(cdiv(M, RBM)), block(256);
+  // one workgroup per panel, and while the panels alone leave the chip (512 slots) half empty, the
+  // panel's column tiles dealt to several, each of which loads and splits the panel again (the
+  // rule of the fused radial-gather kernels, radial_gather.hip)
+  const unsigned panels = cdiv(M, RBM), tiles = cdiv(N, 128);
+  unsigned parts = 1;
+  while (2 * parts <= tiles && panels * parts < 384) parts *= 2;
+  const dim3 grid(panels, parts), block(256);
   hipStream_t s = as_stream(stream);
   // 16-byte output pieces when every row and column group of 4 is aligned
   const bool vec = N % 4 == 0 && ldy % 4 == 0 && aligned16(Y) && (!bias || aligned16(bias));

@@ -98,7 +98,8 @@ __global__ __launch_bounds__(256, 2) void radial_gather_kernel(
     bid[0][g8] = (int32_t)batch[nid[0][g8]];
     bid[1][g8] = (int32_t)batch[nid[1][g8]];
   }
-  for (int t = 0; t < NT; ++t) {
+  const int per = NT / (int)gridDim.y, t0 = per * (int)blockIdx.y;
+  for (int t = t0; t < t0 + per; ++t) {
     // tile t: side so, channel group cg, the radial blocks of degrees 0, 1 (hq 0) or 2 (hq 1)
     const int so = t >> 3, cg = (t >> 1) & 3, hq = t & 1;
     int cb[3];
@@ -256,7 +257,8 @@ __global__ __launch_bounds__(256, 2) void radial_gather_lmax_kernel(
     bid[0][g8] = (int32_t)batch[nid[0][g8]];
     bid[1][g8] = (int32_t)batch[nid[1][g8]];
   }
-  for (int t = 0; t < NTL; ++t) {
+  const int per = NTL / (int)gridDim.y, t0 = per * (int)blockIdx.y;
+  for (int t = t0; t < t0 + per; ++t) {
     const int g = t % L, cg = (t / L) & 3, so = t / (4 * L);
     int cb[3];
 #pragma unroll
@@ -316,6 +318,19 @@ __global__ __launch_bounds__(256, 2) void radial_gather_lmax_kernel(
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   }
+}
+
+// Grid of the two kernels: one workgroup per panel, and while the panels alone leave the chip
+// (512 slots) half empty, up to most_parts (a divisor of the tile count) workgroups per panel,
+// each walking its part of the tiles; a part loads and splits the panel again, about a tile's
+// time.  Alone, us with one workgroup per panel -> this: lmax 2, 870 edges 83 -> 12, 4,500 edges
+// 84 -> 27, 18,000 edges 97 -> 86, 30,000 edges 120 -> 114 (940 workgroups: 120); lmax 4, 870
+// edges 179 -> 29, 9,000 edges 201 -> 95, 30,000 edges 251 -> 235.
+static dim3 panel_grid(int64_t E, int most_parts) {
+  const unsigned panels = cdiv(E, RBM);
+  unsigned parts = 1;
+  while (2 * (int)parts <= most_parts && panels * parts < 384) parts *= 2;
+  return dim3(panels, parts);
 }
 
 }  // namespace rg
@@ -385,7 +400,7 @@ extern "C" int fu_radial_gather_fwd_lmax(const float* h2, int64_t ldh, const voi
   const uint4* w2 = static_cast<const uint4*>(W2);
   const float* cinv = reinterpret_cast<const float*>(w2 + resident_frag_vectors(Nc, K));
   const int* summary = reinterpret_cast<const int*>(cinv + resident_cols(Nc)) + resident_cols(Nc);
-  const dim3 grid((unsigned)cdiv(E, rg::RBM)), block(256);
+  const dim3 grid = rg::panel_grid(E, 8), block(256);
   hipStream_t s = as_stream(stream);
   if (lmax == 3)
     hipLaunchKernelGGL(rg::radial_gather_lmax_kernel<3>, grid, block, 0, s, h2, ldh, w2, cinv, summary, bias, x,
@@ -418,7 +433,7 @@ extern "C" int fu_radial_gather_fwd(const float* h2, int64_t ldh, const void* W2
   const uint4* w2 = static_cast<const uint4*>(W2);
   const float* cinv = reinterpret_cast<const float*>(w2 + resident_frag_vectors(Nc, K));
   const int* summary = reinterpret_cast<const int*>(cinv + resident_cols(Nc)) + resident_cols(Nc);
-  const dim3 grid((unsigned)cdiv(E, rg::RBM)), block(256);
+  const dim3 grid = rg::panel_grid(E, rg::NT), block(256);
   hipStream_t s = as_stream(stream);
   if (layout)
     hipLaunchKernelGGL(rg::radial_gather_kernel<1>, grid, block, 0, s, h2, ldh, w2, cinv, summary, bias, x, idx_i,
