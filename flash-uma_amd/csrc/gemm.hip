@@ -948,9 +948,20 @@ __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_k
   }
 }
 
+void launch_short_ln_bwd(const float* A, int64_t lda, const void* W2, float* g_x, int64_t ldgx, int64_t M, int32_t K,
+                         const float* x, int64_t ldx, const float* gamma, const float* beta, const float* mean,
+                         const float* rstd, int32_t G, hipStream_t st);   // gemm_short.hip
+
 }  // namespace fu
 
 using namespace fu;
+
+// Up to these many rows the radial output layers' input gradients (with a pre-split weight) run in
+// the few-row kernel of gemm_short.hip: its 32-row workgroups read the whole weight each, which
+// past that costs more than the 128-row tiles' idle CUs.  Measured, us, tiled / few-row: K = 1,536
+// 61 / 19 at 870 rows, 79 / 59 at 18,000, 82 / 85 at 30,000; K = 384 26 / 9, 31 / 28, 33 / 37;
+// K = 3,072 109 / 32, 145 / 104, 185 / 175.
+constexpr int64_t SHORT_LN_BWD_MAX_ROWS = 24576;
 
 // Rows from which the split mode uses tall (256-row) tiles: below it the 128-row tiles keep
 // more workgroups in flight than the CU count (the node GEMMs have 8,192 rows).
@@ -1246,6 +1257,12 @@ extern "C" int fu_linear_dgrad_ln_silu_bwd(const float* A, int64_t lda, const fl
   if (!x || !gamma || !beta || !mean || !rstd) return set_error(FU_ERR_NULL, "%s: NULL LayerNorm operand", who);
   if (!aligned16(x) || !aligned16(gamma) || !aligned16(beta))
     return set_error(FU_ERR_ALIGN, "%s: x, gamma and beta must be 16-byte aligned", who);
+  if (W2 && M <= SHORT_LN_BWD_MAX_ROWS && K % GBK == 0 && matmul_mode() == FU_MATMUL_SPLIT_F16) {
+    const int64_t go = (int64_t)group * LN_D;
+    launch_short_ln_bwd(A, lda, W2, g_x, ldgx, M, K, x + go, ldx, gamma + go, beta + go, mean + group, rstd + group, G,
+                        as_stream(stream));
+    return check_launch(who);
+  }
   const int64_t bm = linear_tile_rows(M);
   const int64_t total = (M + bm - 1) / bm;
   if (total > 0x7fffffffLL) return set_error(FU_ERR_SHAPE, "%s: M too large", who);

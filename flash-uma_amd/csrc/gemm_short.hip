@@ -125,22 +125,24 @@ __device__ __forceinline__ void split2h_by(const float4& a, const float4& b, flo
 __device__ __forceinline__ f16x8 frag(const uint4& v) { return __builtin_bit_cast(f16x8, v); }
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
-// This wave's partial 32 x 64 tile of a real contraction, unscaled, into red.
+// This wave's partial 32 x (32 NB) tile of a real contraction, unscaled, into red (rows of STR
+// floats), the K range split over W waves.
+template <int W, int NB, int STR>
 __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_tile, int64_t M, float* red) {
   constexpr int S = RSEG;
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int fr = lane & 31, fh = lane >> 5;
-  const int c0 = wave * p.nk / NW, c1 = (wave + 1) * p.nk / NW;
+  const int c0 = wave * p.nk / W, c1 = (wave + 1) * p.nk / W;
   const int64_t row = row0 + fr < M ? row0 + fr : M - 1;   // a row past M: nothing of it is stored
   const float* pa = p.A + row * p.lda + 8 * fh;
-  const uint4* wb = p.W + (int64_t)(2 * n_tile) * p.nk * 192 + lane;
+  const uint4* wb = p.W + (int64_t)(NB * n_tile) * p.nk * 192 + lane;
   const int64_t wj = (int64_t)p.nk * 192;
   const int wbits = p.flags[0];
   const int last = c1 > c0 ? c1 - 1 : 0;
   // chunk k0 + s of a segment, the last one repeated past the wave's range (not multiplied)
   auto chunk = [&](int k0, int s) { return k0 + s < c1 ? k0 + s : last; };
   float4 raw[S][2];
-  uint4 bh[S][2], bl[S][2];   // hi, lo fragments of the two 32-column blocks
+  uint4 bh[S][NB], bl[S][NB];   // hi, lo fragments of the 32-column blocks
   auto load_a = [&](int k0) {
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -152,12 +154,14 @@ __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_til
 #pragma unroll
     for (int s = 0; s < S; ++s)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < NB; ++j) {
         bh[s][j] = wb[j * wj + (int64_t)chunk(k0, s) * 192];
         bl[s][j] = wb[j * wj + (int64_t)chunk(k0, s) * 192 + 64];
       }
   };
-  floatx16 acc[2] = {zero16(), zero16()};
+  floatx16 acc[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) acc[j] = zero16();
   RowScale sc;
   load_a(c0);
   load_b(c0);
@@ -176,7 +180,7 @@ __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_til
       float rs[16];
       row_factors(fac, fh, rs);
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[j][r] *= rs[r];
     }
@@ -186,7 +190,7 @@ __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_til
     const bool two = (wbits & 1) || ((wbits & 2) && __any(low));
     if (two) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < NB; ++j) {
         acc[j] *= F16_LO_UP;
 #pragma unroll
         for (int s = 0; s < S; ++s) bl[s][j] = wb[j * wj + (int64_t)chunk(k0, s) * 192 + 128];
@@ -203,29 +207,29 @@ __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_til
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < NB; ++j)
             acc[j] = mfma_f16(frag(q == 0 ? al[s] : ah[s]), frag(q == 1 ? bl[s][j] : bh[s][j]), acc[j]);
       }
     if (two) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] *= F16_LO_DOWN;
+      for (int j = 0; j < NB; ++j) acc[j] *= F16_LO_DOWN;
     }
 #pragma unroll
     for (int s = 0; s < S; ++s)
       if (k0 + s < c1) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[j] = mfma_f16(frag(ah[s]), frag(bh[s][j]), acc[j]);
+        for (int j = 0; j < NB; ++j) acc[j] = mfma_f16(frag(ah[s]), frag(bh[s][j]), acc[j]);
       }
     if (k0 + S < c1) load_b(k0 + S);
   }
-  float* ws = red + wave * TR * ES;
+  float* ws = red + wave * TR * STR;
   float rs[16];
   row_factors(pow2i(-sc.e), fh, rs);
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const float cs = p.cinv[64 * n_tile + 32 * j + fr];
+  for (int j = 0; j < NB; ++j) {
+    const float cs = p.cinv[32 * NB * n_tile + 32 * j + fr];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) ws[(8 * (r >> 2) + 4 * fh + (r & 3)) * ES + 32 * j + fr] = acc[j][r] * rs[r] * cs;
+    for (int r = 0; r < 16; ++r) ws[(8 * (r >> 2) + 4 * fh + (r & 3)) * STR + 32 * j + fr] = acc[j][r] * rs[r] * cs;
   }
 }
 
@@ -315,10 +319,11 @@ __device__ __forceinline__ void complex_part(const Prob& p, int64_t row0, int n_
 }
 
 // Sum of the waves' partial values at (row, c .. c + 3), in wave order.
+template <int W = NW, int STR = ES>
 __device__ __forceinline__ float4 sum_parts(const float* red, int row, int c) {
-  float4 v = ld4(red + row * ES + c);
+  float4 v = ld4(red + row * STR + c);
 #pragma unroll
-  for (int w = 1; w < NW; ++w) v = v + ld4(red + (w * TR + row) * ES + c);
+  for (int w = 1; w < W; ++w) v = v + ld4(red + (w * TR + row) * STR + c);
   return v;
 }
 
@@ -340,7 +345,7 @@ __device__ __forceinline__ void real_tile(const Prob& p, const Group& g, int blk
   if (!tile_of(p, g, blk, row0, n_tile)) return;
   const int col0 = 64 * n_tile;
   const int C = g.C, n1 = C / 32, L = g.L;
-  real_part(p, row0, n_tile, g.M, red);
+  real_part<NW, 2, ES>(p, row0, n_tile, g.M, red);
   // MODE 1: a thread takes (row, 4 + 4 columns of the gate pair); otherwise (row, 4 columns)
   constexpr int Q = MODE == 1 ? 8 : 16, IT = TR * Q / (64 * NW);
   const int c = (threadIdx.x % Q) * 4;
@@ -482,6 +487,64 @@ __global__ __launch_bounds__(64 * NW, 3) void short_kernel(const Group g) {
   }
 }
 
+// A radial output layer's input gradient with the LayerNorm-SiLU backward of its group in the
+// epilogue (MODE 5 of gemm.hip: the product is the output gradient, the LayerNorm input x is read),
+// on few rows: a workgroup owns 32 whole 128-column rows and 8 waves split K (1,536 at lmax 2, C =
+// 128), whose 96 chunks a workgroup of the tiled kernel walks one by one however few rows there
+// are: 870 rows 61 -> 19 us, 9,000 rows 77 -> 40 (alone).  Bound by each workgroup's read of the
+// whole weight (786 KB at 64 bytes a cycle, 6 us) and its start and end.
+constexpr int LW = 8, LES = 128 + 8;
+struct LnBwd {
+  const float* x;
+  int64_t ldx;
+  const float* gamma;
+  const float* beta;
+  const float* mean;
+  const float* rstd;
+  int32_t G;   // row stride of mean and rstd
+};
+__global__ __launch_bounds__(64 * LW, 2) void short_ln_bwd_kernel(const Prob p, const LnBwd ln, int64_t M) {
+  __shared__ __attribute__((aligned(16))) float red[LW * TR * LES];
+  const int64_t row0 = (int64_t)blockIdx.x * TR;
+  real_part<LW, 4, LES>(p, row0, 0, M, red);
+  constexpr int IT = TR * 32 / (64 * LW), RS = 2 * LW;   // rows at a time: 32 lanes each
+  const int c = (threadIdx.x & 31) * 4;
+  const float4 gm = ld4(ln.gamma + c), bt = ld4(ln.beta + c);
+  float4 x[IT];
+  float mu[IT], rs[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int64_t row = row0 + (threadIdx.x >> 5) + it * RS;
+    const int64_t rc = row < M ? row : M - 1;
+    x[it] = ld4(ln.x + rc * ln.ldx + c);
+    mu[it] = ln.mean[rc * ln.G];
+    rs[it] = ln.rstd[rc * ln.G];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int r = (int)(threadIdx.x >> 5) + it * RS;
+    const float4 go = sum_parts<LW, LES>(red, r, c);
+    float xh[4], gx[4], s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      xh[t] = ((&x[it].x)[t] - mu[it]) * rs[it];
+      const float y = xh[t] * (&gm.x)[t] + (&bt.x)[t], sg = sigmoidf_(y);
+      gx[t] = (&go.x)[t] * (sg + y * sg * (1.0f - sg)) * (&gm.x)[t];
+      s1 += gx[t];
+      s2 += gx[t] * xh[t];
+    }
+    s1 = group_sum<32>(s1);
+    s2 = group_sum<32>(s2);
+    if (row0 + r < M) {
+      float4 o;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) (&o.x)[t] = rs[it] * (gx[t] - (s1 + xh[t] * s2) / 128.0f);
+      st4(p.Y + (row0 + r) * p.ldy + c, o);
+    }
+  }
+}
+
 template <int MODE, int KIND>
 static void launch(Group& g, int count, hipStream_t st) {
   const int m_tiles = (int)((g.M + TR - 1) / TR + 7) / 8 * 8;
@@ -530,9 +593,49 @@ static int pair_check(const char* who, int64_t E, int32_t C, int32_t L, const vo
 }
 
 }  // namespace sg
+
+// fu_linear_dgrad_ln_silu_bwd on few rows (operands checked by the caller).
+void launch_short_ln_bwd(const float* A, int64_t lda, const void* W2, float* g_x, int64_t ldgx, int64_t M, int32_t K,
+                         const float* x, int64_t ldx, const float* gamma, const float* beta, const float* mean,
+                         const float* rstd, int32_t G, hipStream_t st) {
+  sg::Prob p{};
+  sg::real_weight(p, W2, 128, K);
+  p.A = A;
+  p.lda = lda;
+  p.Y = g_x;
+  p.ldy = ldgx;
+  hipLaunchKernelGGL(sg::short_ln_bwd_kernel, dim3(cdiv(M, sg::TR)), dim3(64 * sg::LW), 0, st, p,
+                     sg::LnBwd{x, ldx, gamma, beta, mean, rstd, G}, M);
+}
+
 }  // namespace fu
 
 using namespace fu;
+
+extern "C" int fu_linear_short(const float* A, int64_t lda, const void* W2, const float* bias, float* Y, int64_t ldy,
+                               int64_t M, int32_t N, int32_t K, void* stream) {
+  using namespace fu::sg;
+  const char* who = "fu_linear_short";
+  if (M < 0 || M > (1 << 24) || N <= 0 || N % 64 != 0 || K < 16 || K % 16 != 0 || lda < K || ldy < N)
+    return set_error(FU_ERR_SHAPE, "%s: M=%lld N=%d K=%d (0 <= M <= 2^24, N %% 64 == 0, K %% 16 == 0)", who,
+                     (long long)M, N, K);
+  if (M == 0) return FU_OK;
+  if (!A || !W2 || !Y) return set_error(FU_ERR_NULL, "%s: NULL argument", who);
+  if (!aligned16(A) || !aligned16(W2) || !aligned16(Y) || (bias && !aligned16(bias)) || lda % 4 != 0 || ldy % 4 != 0)
+    return set_error(FU_ERR_ALIGN, "%s: A, W2, bias and Y must be 16-byte aligned, lda and ldy multiples of 4", who);
+  Group g{};
+  g.M = M;
+  g.C = 64;   // unused by the plain epilogue
+  g.L = 2;
+  real_weight(g.p[0], W2, N, K);
+  g.p[0].A = A;
+  g.p[0].lda = lda;
+  g.p[0].bias = bias;
+  g.p[0].Y = Y;
+  g.p[0].ldy = ldy;
+  launch<0, 0>(g, 1, as_stream(stream));
+  return check_launch(who);
+}
 
 extern "C" int fu_so2_pair_fwd(const float* X0, const float* X1, const float* X2, const void* W0, const float* b0,
                                const void* W1, const void* W2, const void* V0, const float* c0, const void* V1,

@@ -54,6 +54,7 @@ SIGNATURES: dict[str, list] = {
     "fu_linear_weight_split_bytes": [I32, I32],
     "fu_linear_weight_split": [P, I64, I32, I32, P, P],
     "fu_linear_resident": [P, I64, P, P, P, I64, I64, I32, I32, P],
+    "fu_linear_short": [P, I64, P, P, P, I64, I64, I32, I32, P],
     "fu_so2_pair_fwd": [P] * 20 + [I64, I32, I32, P],
     "fu_so2_pair_bwd": [P] * 20 + [I64, I32, I32, P],
     "fu_radial_gather_fwd": [P, I64, P, P, P, P, P, P, P, P, P, P, P, P, I64, I64, I64, I32, I32, I32, P],

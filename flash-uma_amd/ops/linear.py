@@ -79,6 +79,25 @@ def gemm_resident(x: torch.Tensor, W2: torch.Tensor, N: int, bias: torch.Tensor 
     return out
 
 
+# Up to this many rows a plain product of at most 64 columns with a pre-split weight runs in the
+# few-row kernel; the tiled kernels compute 128 columns there.  Measured, us, tiled / few-row, K = 640,
+# N = 64 (the Gaussian gradient of the radial trunk): 27 / 8.5 at 870 rows, 32 / 19 at 18,000, 33 /
+# 24 at 30,000, 44 / 40 at 60,000; K = 320 27 / 28 and K = 1,152 80 / 87 at 60,000.
+FEW_ROWS_MAX = 49152
+
+
+def gemm_few_rows(x: torch.Tensor, W: torch.Tensor, W2: torch.Tensor | None, out: torch.Tensor) -> torch.Tensor:
+    """out = x W^T, on the few-row kernel (fu_linear_short, split-fp16 mode, W pre-split as W2, N =
+    64) up to FEW_ROWS_MAX rows, on fu_linear otherwise."""
+    (M, K), N = x.shape, W.shape[0]
+    if (W2 is None or not 0 < M <= FEW_ROWS_MAX or N != 64 or x.stride(0) % 4 or x.data_ptr() % 16
+            or _lib.get_matmul_mode() != _lib.MATMUL_SPLIT_F16):
+        return gemm(x, W, None, out, W2)
+    _lib.call("fu_linear_short", x.data_ptr(), x.stride(0), W2.data_ptr(), None, out.data_ptr(), out.stride(0), M, N, K,
+              _lib.stream_ptr(x.device))
+    return out
+
+
 def complex_weight_split(P: torch.Tensor, Q: torch.Tensor) -> torch.Tensor:
     """The frozen complex weight P + iQ (Nc, Kc each) pre-split for fu_complex_linear's W3
     argument: exact three-way bf16 splits of P, Q and P + Q in MFMA-fragment order, then their

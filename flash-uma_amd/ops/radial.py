@@ -21,7 +21,7 @@ import torch
 
 from . import _lib
 from .constants import LN_EPS
-from .linear import gemm_resident, linear_weight_split, resident_ok
+from .linear import gemm_few_rows, gemm_resident, linear_weight_split, resident_ok
 
 
 def _ln_grouped_fwd(x, tabs, z, isrc, idst, bias, gamma, beta, G, D, eps):
@@ -418,8 +418,8 @@ class _RadialTrunkFn(torch.autograd.Function):
         del g_p2
         g_p1 = _layer1_bwd(gauss, bank, Z, idx_i, idx_j, m1, r1, g_h1)
         del g_h1
-        g_gauss = _gemm(g_p1, bank.W1g_t, None, torch.empty(E, bank.B, device=gauss.device, dtype=torch.float32),
-                        bank._split("W1g_t", lambda K: K % 16 == 0))
+        g_gauss = gemm_few_rows(g_p1, bank.W1g_t, bank._split("W1g_t", lambda K: K % 16 == 0),
+                                torch.empty(E, bank.B, device=gauss.device, dtype=torch.float32))
         return g_gauss, None, None, None, None, None
 
 

@@ -356,6 +356,13 @@ int fu_linear_weight_split(const float* W, int64_t ldw, int32_t N, int32_t K, vo
 int fu_linear_resident(const float* A, int64_t lda, const void* W2, const float* bias, float* Y, int64_t ldy,
                        int64_t M, int32_t N, int32_t K, void* stream);
 
+/* Y[M, N] = A[M, K] W^T (+ bias[N]) for few rows, W pre-split by fu_linear_weight_split; always in
+ * the split-fp16 form.  32 x 64 output tiles whose K range is split over the waves of a workgroup
+ * (fu_so2_pair_fwd).  N a multiple of 64, K of 16; A, W2, bias and Y 16-byte aligned, lda and ldy
+ * multiples of 4; bias may be NULL; 0 <= M <= 2^24. */
+int fu_linear_short(const float* A, int64_t lda, const void* W2, const float* bias, float* Y, int64_t ldy, int64_t M,
+                    int32_t N, int32_t K, void* stream);
+
 /* The SO(2) convolution pair of a block on few edges (model.py:150-154), split-fp16 mode only
  * (FU_ERR_UNSUPPORTED otherwise): conv1 + gate + conv2 in three launches, and their input
  * gradients in three, each 32 x 64 output tile's K range split over the waves of a workgroup.  The

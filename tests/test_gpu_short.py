@@ -1,4 +1,5 @@
-"""The few-row kernels of the SO(2) convolution pair (fu_so2_pair_fwd / _bwd) against float64, at the
+"""The few-row kernels (the SO(2) convolution pair fu_so2_pair_fwd / _bwd, fu_linear_short, and
+fu_linear_dgrad_ln_silu_bwd with a pre-split weight) against float64, at the
 edges of their 32-row tiles, for every lmax and several widths (K ranges that do not divide evenly
 over the waves), and where the fp16 window rule sends a segment to the two-loop products."""
 import pytest
@@ -93,3 +94,55 @@ def test_short_pair_nonfinite_rows_stay_apart(cuda):
     for a, b in zip(got, clean):
         assert torch.equal(a[ok], b[ok])
     assert not torch.isfinite(got[0][3]).all() and not torch.isfinite(got[1][50]).all()
+
+
+@pytest.mark.parametrize("M,N,K,ramp", [(1, 64, 640, 0), (33, 64, 640, 0), (200, 192, 16, 0), (65, 64, 48, 0),
+                                        (90, 128, 1152, 0), (70, 64, 320, 12)])
+def test_linear_short(cuda, M, N, K, ramp):
+    """fu_linear_short on K ranges shorter than and not divisible by its four waves, a strided output
+    whose other columns keep their contents, and anti-correlated magnitudes (the two-loop products);
+    bar as above."""
+    from ops import _lib, linear
+    g = torch.Generator().manual_seed(M + N + K)
+    f = torch.exp2(torch.round(torch.linspace(-ramp, ramp, K)))
+    x, W, b = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5, torch.randn(N, generator=g)
+    ref = x.double() @ W.double().T + b.double()
+    xd, Wd, bd = (x * f).to(cuda), (W / f).to(cuda), b.to(cuda)
+    W2 = linear.linear_weight_split(Wd)
+    buf = torch.full((M, N + 4), 7.0, device=cuda)
+    _lib.call("fu_linear_short", xd.data_ptr(), K, W2.data_ptr(), bd.data_ptr(), buf.data_ptr(), N + 4, M, N, K,
+              _lib.stream_ptr(cuda))
+    tiled = linear.gemm(xd, Wd, bd)
+    e, t = _err([buf[:, :N], tiled], [ref, ref])
+    assert (buf[:, N:] == 7.0).all() and e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
+
+
+@pytest.mark.parametrize("M,K,group", [(1, 1536, 0), (31, 384, 4), (33, 1536, 2), (500, 3072, 1), (70, 16, 3)])
+def test_dgrad_ln_silu_short(cuda, M, K, group):
+    """The radial output layer's input gradient with the LayerNorm-SiLU backward of its group, few rows
+    and a pre-split weight, against float64 and the tiled kernel (no pre-split weight); the other
+    groups' columns keep their contents."""
+    from ops import _lib, linear
+    G, C = 5, 128
+    g = torch.Generator(device=cuda).manual_seed(M + K)
+    r = lambda *s: torch.randn(*s, device=cuda, generator=g)
+    A, W, x = r(M, K), r(C, K) / K ** 0.5, r(M, G * C)
+    gm, bt = r(G * C).abs() + 0.5, r(G * C) * 0.1
+    xd = x.double().view(M, G, C)
+    mean, var = xd.mean(2), xd.var(2, unbiased=False)
+    mu, rs = mean.float().flatten().contiguous(), (var + 1e-5).rsqrt().float().flatten().contiguous()
+    W2, s = linear.linear_weight_split(W), slice(group * C, (group + 1) * C)
+    outs = []
+    for w2 in (W2, None):
+        out = torch.full((M, G * C), 7.0, device=cuda)
+        _lib.call("fu_linear_dgrad_ln_silu_bwd", A.data_ptr(), K, W.data_ptr(), K, out[:, s].data_ptr(), G * C, M, K,
+                  x.data_ptr(), G * C, gm.data_ptr(), bt.data_ptr(), mu.data_ptr(), rs.data_ptr(), G, group,
+                  _lib.ptr(w2), _lib.stream_ptr(cuda))
+        assert (out[:, :s.start] == 7.0).all() and (out[:, s.stop:] == 7.0).all()
+        outs.append(out[:, s])
+    v = x[:, s].double().requires_grad_()
+    xh = (v - v.mean(1, keepdim=True)) * (v.var(1, unbiased=False, keepdim=True) + 1e-5).rsqrt()
+    y = torch.nn.functional.silu(xh * gm[s].double() + bt[s].double())
+    (ref,) = torch.autograd.grad(y, v, A.double() @ W.double().T)
+    e, t = _err(outs, [ref.cpu()] * 2)
+    assert e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
