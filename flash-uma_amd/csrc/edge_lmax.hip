@@ -18,9 +18,10 @@
 // gives rows m = -2..2 of D^3 (5 x 7) and D^4 (5 x 9).
 //
 // Mapping (HBM-bound, like the lmax = 2 kernels): forward gather and backward scatter one
-// wave64 per edge, lanes across channels, a contiguous XCD-aware edge range per workgroup; forward scatters one wave per receiver with fp64
-// accumulators, segments in CSR order; backward gather node-centric (one wave per CSR
-// segment of the node, as receiver and as sender), so no kernel uses atomics.  The l blocks
+// wave64 per edge, lanes across channels, a contiguous XCD-aware edge range per workgroup; forward
+// scatters one wave per receiver with fp64 accumulators, segments in CSR order; backward gather
+// node-centric (one wave per CSR segment of the node, as receiver and as sender), so no kernel uses
+// atomics.  With few nodes two or four waves share a segment (node_waves, segment_waves).  The l blocks
 // are processed one at a time to bound registers.
 #include "edge_lmax_layout.h"
 #include "fu_vec.h"
@@ -224,16 +225,18 @@ __device__ __forceinline__ void gather_bwd_block(const float* sv, const float* w
   reduce_store<nr * nk>(part, gw_l, lane, accw);
 }
 
-template <int CPL, int L>
+template <int CPL, int L, int W>
 __device__ __forceinline__ void gather_bwd_segment(const float* __restrict__ gX0, const float* __restrict__ gX1,
                                                    const float* __restrict__ gX2, const float* __restrict__ wig,
                                                    const float* __restrict__ ext, const float* __restrict__ rad,
                                                    const int32_t* __restrict__ ptr, const int32_t* __restrict__ idx,
-                                                   int64_t n, int so, const float* sv, Vec<CPL> (&acc)[ncoef(L)],
-                                                   float* __restrict__ g_rad, float* __restrict__ gw,
-                                                   float* __restrict__ gext, int c, int lane, bool accw) {
+                                                   int64_t n, int so, int part, const float* sv,
+                                                   Vec<CPL> (&acc)[ncoef(L)], float* __restrict__ g_rad,
+                                                   float* __restrict__ gw, float* __restrict__ gext, int c, int lane,
+                                                   bool accw) {
   constexpr int C = 64 * CPL, EW = extw(L);
-  const int32_t k0 = ptr[n], k1 = ptr[n + 1];
+  int32_t k0 = ptr[n], k1 = ptr[n + 1];
+  segment_part<W>(part, k0, k1);
   for (int32_t k = k0; k < k1; ++k) {
     const int64_t e = idx[k];
     const float* wl = wig + e * 34;
@@ -260,11 +263,12 @@ __device__ __forceinline__ void gather_bwd_segment(const float* __restrict__ gX0
   }
 }
 
-// One node per 128-thread workgroup: wave 0 walks the receiver segment, wave 1 the sender
-// segment; each wave keeps its own LDS copy of the node row (csd added on l = 0), the two
-// node-gradient partials meet in LDS and g_x[n] is written once.
-template <int CPL, int L>
-__global__ __launch_bounds__(128) void gather_bwd_lmax_kernel(
+// One node per workgroup, W waves per segment (segment_waves): the first W walk parts of the
+// receiver segment, the others of the sender segment; each wave (W = 1), or the workgroup, keeps an
+// LDS copy of the node row (csd added on l = 0); the node-gradient partials meet in LDS, are added
+// in part order (receiver first) and g_x[n] is written once.
+template <int CPL, int L, int W>
+__global__ __launch_bounds__(128 * W) void gather_bwd_lmax_kernel(
     const float* __restrict__ gX0, const float* __restrict__ gX1, const float* __restrict__ gX2,
     const float* __restrict__ x, const float* __restrict__ wig, const float* __restrict__ ext,
     const float* __restrict__ rad, const float* __restrict__ csd, const int64_t* __restrict__ batch,
@@ -273,8 +277,8 @@ __global__ __launch_bounds__(128) void gather_bwd_lmax_kernel(
     float* __restrict__ gext_recv, float* __restrict__ gw_send, float* __restrict__ gext_send,
     float* __restrict__ g_rad, int64_t N, int32_t acc_flags) {
   constexpr int C = 64 * CPL, K = ncoef(L);
-  __shared__ __attribute__((aligned(16))) float s_v[2][K * C];
-  __shared__ __attribute__((aligned(16))) float s_send[K * C];
+  __shared__ __attribute__((aligned(16))) float s_v[W == 1 ? 2 : 1][K * C];
+  __shared__ __attribute__((aligned(16))) float s_part[2 * W - 1][K * C];
   const int lane = threadIdx.x & 63;
   const int wave = wave_uniform();
   const int64_t n = (int64_t)blockIdx.x;
@@ -282,31 +286,39 @@ __global__ __launch_bounds__(128) void gather_bwd_lmax_kernel(
   Vec<CPL> acc[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) acc[k] = vzero<CPL>();
-  float* sv = s_v[wave];
+  float* sv = s_v[W == 1 ? wave : 0];
   const float* xn = x + n * K * C + c;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
+    if (W > 1 && k % (2 * W) != wave) continue;
     Vec<CPL> r = vload<CPL>(xn + k * C);
     if (k == 0) r = vadd(r, vload<CPL>(csd + batch[n] * C + c));
     vstore(sv + k * C + c, r);
   }
-  if (wave == 0) {
-    // the receiver half goes into the caller's g_wigner / g_wig_ext (added to their contents
-    // when accumulating: only this wave writes an edge's entries there), the sender half into
-    // the workspace, added afterwards
-    gather_bwd_segment<CPL, L>(gX0, gX1, gX2, wig, ext, rad, rptr, ridx, n, 1, sv, acc, g_rad, gw_recv, gext_recv, c,
-                               lane, (acc_flags & 1) != 0);
-  } else {
-    gather_bwd_segment<CPL, L>(gX0, gX1, gX2, wig, ext, rad, sptr, sidx, n, 0, sv, acc, g_rad, gw_send, gext_send, c,
-                               lane, false);
+  if constexpr (W > 1) __syncthreads();
+  // the receiver half goes into the caller's g_wigner / g_wig_ext (added to their contents when
+  // accumulating: only one wave writes an edge's entries there), the sender half into the
+  // workspace, added afterwards
+  if (wave < W)
+    gather_bwd_segment<CPL, L, W>(gX0, gX1, gX2, wig, ext, rad, rptr, ridx, n, 1, wave, sv, acc, g_rad, gw_recv,
+                                  gext_recv, c, lane, (acc_flags & 1) != 0);
+  else
+    gather_bwd_segment<CPL, L, W>(gX0, gX1, gX2, wig, ext, rad, sptr, sidx, n, 0, wave - W, sv, acc, g_rad, gw_send,
+                                  gext_send, c, lane, false);
+  if (wave > 0) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) vstore(&s_send[k * C + c], acc[k]);
+    for (int k = 0; k < K; ++k) vstore(&s_part[wave - 1][k * C + c], acc[k]);
   }
   __syncthreads();
   if (wave == 0) {
     float* gx = g_x + n * K * C + c;
 #pragma unroll
-    for (int k = 0; k < K; ++k) vstore(gx + k * C, vadd(acc[k], vload<CPL>(&s_send[k * C + c])));
+    for (int k = 0; k < K; ++k) {
+      Vec<CPL> t = acc[k];
+#pragma unroll
+      for (int w = 0; w < 2 * W - 1; ++w) t = vadd(t, vload<CPL>(&s_part[w][k * C + c]));
+      vstore(gx + k * C, t);
+    }
   }
 }
 
@@ -338,7 +350,8 @@ __device__ __forceinline__ void scatter_fwd_block(const float* wl, const float* 
   }
 }
 
-template <int CPL, int L>
+// W waves per node (node_waves).
+template <int CPL, int L, int W>
 __global__ __launch_bounds__(256) void scatter_fwd_lmax_kernel(
     const int32_t* __restrict__ rptr, const int32_t* __restrict__ col, const float* __restrict__ Z0,
     const float* __restrict__ Z1, const float* __restrict__ Z2, const float* __restrict__ wig,
@@ -347,17 +360,23 @@ __global__ __launch_bounds__(256) void scatter_fwd_lmax_kernel(
   constexpr int C = 64 * CPL, K = ncoef(L), EW = extw(L);
   const int lane = threadIdx.x & 63;
   const int c = lane * CPL;
-  const int64_t n = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave_uniform();
-  if (n >= N) return;
+  __shared__ double s_acc[W > 1 ? (4 / W) * (W - 1) * K * C : 1];
+  const int local = wave_uniform() / W, part = wave_uniform() % W;
+  const int64_t n = (int64_t)blockIdx.x * (4 / W) + local;
+  if (W == 1 && n >= N) return;   // with several waves per node every wave reaches the barrier
+  const bool live = n < N;
   double acc[K][CPL];
   const float* xr = x_res + n * K * C + c;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const Vec<CPL> t = vload<CPL>(xr + k * C);
+    Vec<CPL> t = vzero<CPL>();
+    if (W == 1 || (live && part == 0)) t = vload<CPL>(xr + k * C);
 #pragma unroll
     for (int q = 0; q < CPL; ++q) acc[k][q] = (double)t[q];
   }
-  for (int32_t k = rptr[n]; k < rptr[n + 1]; ++k) {
+  int32_t k0 = live ? rptr[n] : 0, k1 = live ? rptr[n + 1] : 0;
+  segment_part<W>(part, k0, k1);
+  for (int32_t k = k0; k < k1; ++k) {
     const int64_t e = col[k];
     const float en = env[e];
     const float* wl = wig + e * 34;
@@ -373,6 +392,8 @@ __global__ __launch_bounds__(256) void scatter_fwd_lmax_kernel(
     if constexpr (L >= 3) scatter_fwd_block<L, CPL, 3>(wl, we, en, Z0e, Z1e, Z2e, acc);
     if constexpr (L >= 4) scatter_fwd_block<L, CPL, 4>(wl, we, en, Z0e, Z1e, Z2e, acc);
   }
+  add_parts<W, CPL, K>(s_acc, local, part, lane, acc);
+  if (W > 1 && (!live || part > 0)) return;
   float* xo = x_out + n * K * C + c;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -816,9 +837,12 @@ extern "C" int fu_gather_bwd_lmax(const float* g_X_m0, const float* g_X_m1, cons
   float* ws_x = ws + E * 34;
   with_c_lmax(C, lmax, [&](auto cpl, auto lv) {
     constexpr int P = decltype(cpl)::value, L = decltype(lv)::value;
-    hipLaunchKernelGGL((gather_bwd_lmax_kernel<P, L>), dim3((unsigned)N), dim3(128), 0, s, g_X_m0, g_X_m1, g_X_m2, x,
-                       wigner, wig_ext, rad, csd_emb, batch, recv_ptr, recv_idx, send_ptr, send_idx, g_x, g_wigner,
-                       g_wig_ext, ws_w, ws_x, g_rad, N, accumulate);
+    with_waves<P>(segment_waves(N), [&](auto w) {
+      constexpr int W = decltype(w)::value;
+      hipLaunchKernelGGL((gather_bwd_lmax_kernel<P, L, W>), dim3((unsigned)N), dim3(128 * W), 0, s, g_X_m0, g_X_m1,
+                         g_X_m2, x, wigner, wig_ext, rad, csd_emb, batch, recv_ptr, recv_idx, send_ptr, send_idx, g_x,
+                         g_wigner, g_wig_ext, ws_w, ws_x, g_rad, N, accumulate);
+    });
   });
   st = check_launch("fu_gather_bwd_lmax");
   if (st != FU_OK || E == 0) return st;
@@ -844,8 +868,11 @@ extern "C" int fu_scatter_fwd_lmax(const int32_t* row_ptr, const int32_t* col_id
   hipStream_t s = as_stream(stream);
   with_c_lmax(C, lmax, [&](auto cpl, auto lv) {
     constexpr int P = decltype(cpl)::value, L = decltype(lv)::value;
-    hipLaunchKernelGGL((scatter_fwd_lmax_kernel<P, L>), dim3(cdiv(N, 4)), dim3(256), 0, s, row_ptr, col_idx, Z_m0,
-                       Z_m1, Z_m2, wigner, wig_ext, env, x_res, x_out, N);
+    with_waves<P>(node_waves(N), [&](auto w) {
+      constexpr int W = decltype(w)::value;
+      hipLaunchKernelGGL((scatter_fwd_lmax_kernel<P, L, W>), dim3(cdiv(N, 4 / W)), dim3(256), 0, s, row_ptr, col_idx,
+                         Z_m0, Z_m1, Z_m2, wigner, wig_ext, env, x_res, x_out, N);
+    });
   });
   return check_launch("fu_scatter_fwd_lmax");
 }

@@ -176,4 +176,66 @@ __device__ __forceinline__ float wave_multi_sum(const float (&vals)[V], int lane
   return r;
 }
 
+// Waves that share one node's segment in the forward scatters.  With few nodes one wave walks its
+// 30 to 60 edges one after the other at the latency of their loads while most of the chip is idle, so
+// two or four waves take contiguous parts of the segment and their fp64 sums are added in part order.
+// us at C = 128, bcc segments of about 38 edges, for 1 | 2 | 4 waves:
+//   nodes                      54            300           1000          1500           3000
+//   rotate_scatter, lmax 2   22|13| 9      27|17|13      34|29|28      47| 42| 44     77| 84| 83
+//   init_scatter,   lmax 2   11| 8| 7      13| 9| 8      18|14|13      23| 17| 19     32| 31| 34
+//   rotate_scatter, lmax 4   45|27|16      80|50|29     123|94|87     149|114|126    199|219|244
+inline int node_waves(int64_t N) { return N <= 1024 ? 4 : N <= 1536 ? 2 : 1; }
+
+// The part of wave `part` of W of the CSR segment [k0, k1).
+template <int W>
+__device__ __forceinline__ void segment_part(int part, int32_t& k0, int32_t& k1) {
+  if constexpr (W > 1) {
+    const int32_t a = k0, len = k1 - k0;
+    k0 = a + (int32_t)((int64_t)len * part / W);
+    k1 = a + (int32_t)((int64_t)len * (part + 1) / W);
+  }
+}
+
+// acc of part 0 += the other parts', in part order (every wave of the workgroup calls this; the
+// result is in part 0)
+template <int W, int CPL, int K>
+__device__ __forceinline__ void add_parts(double* s_acc, int node_local, int part, int lane, double (&acc)[K][CPL]) {
+  if constexpr (W > 1) {
+    constexpr int C = 64 * CPL;
+    double* mine = s_acc + (int64_t)(node_local * (W - 1) + (part > 0 ? part - 1 : 0)) * K * C + lane;
+    if (part > 0) {
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int q = 0; q < CPL; ++q) mine[k * C + 64 * q] = acc[k][q];
+    }
+    __syncthreads();
+    if (part == 0) {
+#pragma unroll
+      for (int w = 0; w < W - 1; ++w)
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int q = 0; q < CPL; ++q) acc[k][q] += mine[(w * K + k) * C + 64 * q];
+    }
+  }
+}
+
+// f(w) for w = 1, 2 or 4 waves; one at C = 256 (CPL 4), whose rows fill the registers and LDS
+template <int CPL, typename F>
+inline void with_waves(int w, F f) {
+  if constexpr (CPL < 4) {
+    if (w == 4) return f(std::integral_constant<int, 4>{});
+    if (w == 2) return f(std::integral_constant<int, 2>{});
+  }
+  f(std::integral_constant<int, 1>{});
+}
+
+// Waves per segment of the gather backward, whose block already holds a wave per side; the rows of four
+// a side hold 154 KB of LDS at lmax 4, so only one block fits a CU.  As above:
+//   nodes                      54            150           500           1000          1500
+//   lmax 2                   47|28|25      49| 31|29     77| 72| 73    145|136|136   206|201|198
+//   lmax 4                 163|92|73     172|101|80    225|161|179    297|296|338   499|431|487
+inline int segment_waves(int64_t N) { return N <= 256 ? 4 : N <= 2048 ? 2 : 1; }
+
 }  // namespace fu

@@ -9,7 +9,8 @@
 //
 // Backward: node-centric.  A 128-thread workgroup owns one node: one wave walks the node's
 // receiver segment (edges e with idx_j[e] = n, receiver CSR) and the other its sender
-// segment (idx_i[e] = n, sender CSR).  Each wave recomputes the rotated own row,
+// segment (idx_i[e] = n, sender CSR); with few nodes two or four waves share each segment
+// (segment_waves).  Each wave recomputes the rotated own row,
 // writes its half of g_rad, accumulates D^T g into the node gradient in CSR order, and
 // reduces its half of g_wigner across lanes.  The two node partials are added through LDS
 // (receiver part + sender part) and g_x[n] is written once: deterministic, no atomics.
@@ -305,18 +306,19 @@ __device__ __forceinline__ void side_apply(const SideEdge<CPL>& d, int64_t e, in
   }
 }
 
-// One side of one node's gather backward: walk the node's CSR segment in order.  The
+// One side of one node's gather backward: walk part `part` of W of the node's CSR segment in order.  The
 // segment's edge ids are fetched 64 at a time into one VGPR (lane t holds the t-th id) and
 // broadcast with readlane; the loads of edge t+1 are issued before edge t is processed.
-template <int CPL, int L>
+template <int CPL, int L, int W>
 __device__ __forceinline__ void gather_bwd_side(const float* __restrict__ gX0, const float* __restrict__ gX1,
                                                 const float* __restrict__ gX2, const float* __restrict__ wig,
                                                 const float* __restrict__ rad, const int32_t* __restrict__ ptr,
-                                                const int32_t* __restrict__ idx, int64_t n, int so, const float* sv,
-                                                Rows9<CPL>& acc, float* __restrict__ g_rad,
+                                                const int32_t* __restrict__ idx, int64_t n, int so, int part,
+                                                const float* sv, Rows9<CPL>& acc, float* __restrict__ g_rad,
                                                 float* __restrict__ gw_out, int lane, bool accw) {
   const int c = lane * CPL;
-  const int32_t k0 = ptr[n], k1 = ptr[n + 1];
+  int32_t k0 = ptr[n], k1 = ptr[n + 1];
+  segment_part<W>(part, k0, k1);
   for (int32_t base = k0; base < k1; base += 64) {
     const int cnt = (int)std::min<int32_t>(64, k1 - base);
     const int32_t ids = lane < cnt ? idx[base + lane] : 0;
@@ -349,53 +351,58 @@ __device__ __forceinline__ void gather_bwd_side(const float* __restrict__ gX0, c
 // C = 256 two edges in flight need more than the 170 registers of 3 waves per SIMD (449
 // spilled to scratch) or the 256 of 2 (116): one wave per SIMD keeps them in registers and
 // accumulation registers (2.26x faster at 245,760 edges: 5,160 -> 2,285 us).
-template <int CPL, int L>
-__global__ __launch_bounds__(128, CPL >= 4 ? 1 : 3) void gather_bwd_kernel(
+// W waves per segment (node_waves below): with few nodes each takes a contiguous part of the
+// segment, and the node gradients are added in part order, receiver parts first.
+template <int CPL, int L, int W>
+__global__ __launch_bounds__(128 * W, CPL >= 4 ? 1 : 3) void gather_bwd_kernel(
     const float* __restrict__ gX0, const float* __restrict__ gX1, const float* __restrict__ gX2,
     const float* __restrict__ x, const float* __restrict__ wig, const float* __restrict__ rad,
     const float* __restrict__ csd, const int64_t* __restrict__ batch, const int32_t* __restrict__ rptr,
     const int32_t* __restrict__ ridx, const int32_t* __restrict__ sptr, const int32_t* __restrict__ sidx,
     float* __restrict__ g_x, float* __restrict__ g_wig, float* __restrict__ g_rad, float* __restrict__ ws,
-    int64_t N, int32_t acc_flags) {
+    int32_t acc_flags) {
   constexpr int C = 64 * CPL;
-  __shared__ __attribute__((aligned(16))) float s_send[1][9 * C];
-  __shared__ __attribute__((aligned(16))) float s_v[2][9 * C];
+  __shared__ __attribute__((aligned(16))) float s_part[2 * W - 1][9 * C];
+  __shared__ __attribute__((aligned(16))) float s_v[2 * W][9 * C];
   const int lane = threadIdx.x & 63;
   const int wave = wave_id_uniform();
-  const int node_local = 0;
-  const int side = wave;  // 0: receiver segment, 1: sender segment
+  const int side = wave / W, part = wave % W;  // side 0: receiver segment, 1: sender segment
   const int64_t n = (int64_t)blockIdx.x;
   const int c = lane * CPL;
   Rows9<CPL> acc;
 #pragma unroll
   for (int k = 0; k < 9; ++k) acc.r[k] = vzero<CPL>();
-  if (n < N) {
-    // the node's own row (csd added on l = 0) in this wave's LDS slot; each lane reads back
-    // only the channels it wrote, so no barrier is needed
-    float* sv = s_v[wave];
-    const float* xn = x + n * 9 * C + c;
+  // the node's own row (csd added on l = 0) in this wave's LDS slot; each lane reads back only
+  // the channels it wrote, so no barrier is needed
+  float* sv = s_v[wave];
+  const float* xn = x + n * 9 * C + c;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      Vec<CPL> r = vload<CPL>(xn + k * C);
-      if (k == 0) r = vadd(r, vload<CPL>(csd + batch[n] * C + c));
-      vstore(sv + k * C + c, r);
-    }
-    if (side == 0) {
-      // receiver half into g_wigner (added to its contents when accumulating: only this wave
-      // writes an edge's entries there); sender half into the workspace, added afterwards
-      gather_bwd_side<CPL, L>(gX0, gX1, gX2, wig, rad, rptr, ridx, n, 1, sv, acc, g_rad, g_wig, lane,
-                              (acc_flags & 1) != 0);
-    } else {
-      gather_bwd_side<CPL, L>(gX0, gX1, gX2, wig, rad, sptr, sidx, n, 0, sv, acc, g_rad, ws, lane, false);
+  for (int k = 0; k < 9; ++k) {
+    Vec<CPL> r = vload<CPL>(xn + k * C);
+    if (k == 0) r = vadd(r, vload<CPL>(csd + batch[n] * C + c));
+    vstore(sv + k * C + c, r);
+  }
+  // receiver half into g_wigner (added to its contents when accumulating: only one wave writes an
+  // edge's entries there); sender half into the workspace, added afterwards
+  if (side == 0)
+    gather_bwd_side<CPL, L, W>(gX0, gX1, gX2, wig, rad, rptr, ridx, n, 1, part, sv, acc, g_rad, g_wig, lane,
+                               (acc_flags & 1) != 0);
+  else
+    gather_bwd_side<CPL, L, W>(gX0, gX1, gX2, wig, rad, sptr, sidx, n, 0, part, sv, acc, g_rad, ws, lane, false);
+  if (wave > 0) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) vstore(&s_send[node_local][k * C + c], acc.r[k]);
-    }
+    for (int k = 0; k < 9; ++k) vstore(&s_part[wave - 1][k * C + c], acc.r[k]);
   }
   __syncthreads();
-  if (n < N && side == 0) {
+  if (wave == 0) {
     float* gx = g_x + n * 9 * C + c;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) vstore(gx + k * C, vadd(acc.r[k], vload<CPL>(&s_send[node_local][k * C + c])));
+    for (int k = 0; k < 9; ++k) {
+      Vec<CPL> t = acc.r[k];
+#pragma unroll
+      for (int w = 0; w < 2 * W - 1; ++w) t = vadd(t, vload<CPL>(&s_part[w][k * C + c]));
+      vstore(gx + k * C, t);
+    }
   }
 }
 
@@ -431,8 +438,11 @@ static void launch_gather_bwd(const float* gX0, const float* gX1, const float* g
                               const int32_t* rptr, const int32_t* ridx, const int32_t* sptr, const int32_t* sidx,
                               float* g_x, float* g_wig, float* g_rad, float* ws, int64_t N, int32_t acc,
                               hipStream_t st) {
-  hipLaunchKernelGGL((gather_bwd_kernel<CPL, L>), dim3((unsigned)N), dim3(128), 0, st, gX0, gX1, gX2, x, wigner, rad, csd,
-                     batch, rptr, ridx, sptr, sidx, g_x, g_wig, g_rad, ws, N, acc);
+  with_waves<CPL>(segment_waves(N), [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((gather_bwd_kernel<CPL, L, W>), dim3((unsigned)N), dim3(128 * W), 0, st, gX0, gX1, gX2, x, wigner,
+                       rad, csd, batch, rptr, ridx, sptr, sidx, g_x, g_wig, g_rad, ws, acc);
+  });
 }
 
 }  // namespace fu

@@ -2,9 +2,10 @@
 // (ops/scatter.py:45-140), the edge-degree embedding scatter (ops/scatter.py:360-423) and
 // both backward passes (ops/scatter.py:146-292, 426-481).
 //
-// Forward kernels: one wave64 per receiver node, lanes across channels; the node's CSR
-// segment is walked in order and every edge message (computed in fp32 exactly as the
-// reference forms it) is accumulated into fp64 registers, then rounded once to fp32.
+// Forward kernels: one wave64 per receiver node (two or four when nodes are few: node_waves),
+// lanes across channels; the node's CSR segment is walked in order and every edge message
+// (computed in fp32 exactly as the reference forms it) is accumulated into fp64 registers, then
+// rounded once to fp32.
 // Backward kernels: one wave64 per edge, contiguous XCD-aware edge range per workgroup
 // (block_edge_range); the per-edge channel reductions for g_wigner and g_env use one
 // multi-value wave reduction.
@@ -36,7 +37,8 @@ __device__ __forceinline__ void load_zr(const float* Z0, const float* Z1, const 
   zr[4] = vload_nt<CPL>(z2 + C);
 }
 
-template <int CPL>
+// W waves per node (node_waves).
+template <int CPL, int W>
 __global__ __launch_bounds__(256) void scatter_fwd_kernel(const int32_t* __restrict__ rptr,
                                                           const int32_t* __restrict__ col,
                                                           const float* __restrict__ Z0, const float* __restrict__ Z1,
@@ -47,17 +49,22 @@ __global__ __launch_bounds__(256) void scatter_fwd_kernel(const int32_t* __restr
   constexpr int C = 64 * CPL;
   const int lane = threadIdx.x & 63;
   const int c = lane * CPL;
-  const int64_t n = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave_id_u();
-  if (n >= N) return;
+  __shared__ double s_acc[W > 1 ? (4 / W) * (W - 1) * 9 * C : 1];
+  const int local = wave_id_u() / W, part = wave_id_u() % W;
+  const int64_t n = (int64_t)blockIdx.x * (4 / W) + local;
+  if (W == 1 && n >= N) return;   // with several waves per node every wave reaches the barrier
+  const bool live = n < N;
   double acc[9][CPL];
   const float* xr = x_res + n * 9 * C + c;
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    const Vec<CPL> t = vload<CPL>(xr + k * C);
+    Vec<CPL> t = vzero<CPL>();
+    if (W == 1 || (live && part == 0)) t = vload<CPL>(xr + k * C);
 #pragma unroll
     for (int q = 0; q < CPL; ++q) acc[k][q] = (double)t[q];
   }
-  const int32_t k0 = rptr[n], k1 = rptr[n + 1];
+  int32_t k0 = live ? rptr[n] : 0, k1 = live ? rptr[n + 1] : 0;
+  segment_part<W>(part, k0, k1);
   // one edge's message env * D^T zr, accumulated into the fp64 registers
   auto accumulate = [&](const float* w, float en, const Vec<CPL>(&zr)[9]) {
 #pragma unroll
@@ -103,6 +110,8 @@ __global__ __launch_bounds__(256) void scatter_fwd_kernel(const int32_t* __restr
     }
     if (k < k1) accumulate(wa, ena, za);
   }
+  add_parts<W, CPL, 9>(s_acc, local, part, lane, acc);
+  if (W > 1 && (!live || part > 0)) return;
   float* xo = x_out + n * 9 * C + c;
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(256) void scatter_bwd_kernel(const float* __restric
   }
 }
 
-template <int CPL>
+template <int CPL, int W>
 __global__ __launch_bounds__(256) void init_scatter_fwd_kernel(
     const int32_t* __restrict__ rptr, const int32_t* __restrict__ col, const float* __restrict__ rad,
     const float* __restrict__ wig, const float* __restrict__ env, const int64_t* __restrict__ Z,
@@ -206,19 +215,24 @@ __global__ __launch_bounds__(256) void init_scatter_fwd_kernel(
   constexpr int C = 64 * CPL;
   const int lane = threadIdx.x & 63;
   const int c = lane * CPL;
-  const int64_t n = (int64_t)blockIdx.x * (blockDim.x >> 6) + wave_id_u();
-  if (n >= N) return;
+  __shared__ double s_acc[W > 1 ? (4 / W) * (W - 1) * 9 * C : 1];
+  const int local = wave_id_u() / W, part = wave_id_u() % W;
+  const int64_t n = (int64_t)blockIdx.x * (4 / W) + local;
+  if (W == 1 && n >= N) return;
+  const bool live = n < N;
   double acc[9][CPL], base[CPL];
-  {
+#pragma unroll
+  for (int q = 0; q < CPL; ++q) base[q] = 0.0;
+  if (W == 1 || live) {
     const Vec<CPL> ws = vload<CPL>(W_sphere + Z[n] * C + c);
     const Vec<CPL> cs = vload<CPL>(csd + batch[n] * C + c);
 #pragma unroll
     for (int q = 0; q < CPL; ++q) base[q] = (double)(ws[q] + cs[q]);
-#pragma unroll
-    for (int k = 0; k < 9; ++k)
-#pragma unroll
-      for (int q = 0; q < CPL; ++q) acc[k][q] = 0.0;
   }
+#pragma unroll
+  for (int k = 0; k < 9; ++k)
+#pragma unroll
+    for (int q = 0; q < CPL; ++q) acc[k][q] = 0.0;
   // The receiver's edges in CSR order; the next edge's loads are issued before the current
   // edge is accumulated (two register sets, sched_barrier keeping the scheduler from sinking
   // them), since one edge's arithmetic is short next to its load latency.
@@ -249,7 +263,8 @@ __global__ __launch_bounds__(256) void init_scatter_fwd_kernel(
       for (int b = 0; b < 5; ++b) acc[4 + b][q] += (double)(d.r[2][q] * d.w2[b] * d.en);
     }
   };
-  const int32_t k0 = rptr[n], k1 = rptr[n + 1];
+  int32_t k0 = live ? rptr[n] : 0, k1 = live ? rptr[n + 1] : 0;
+  segment_part<W>(part, k0, k1);
   if (k0 < k1) {
     EdgeData d0, d1;
     load(k0, d0);
@@ -266,6 +281,8 @@ __global__ __launch_bounds__(256) void init_scatter_fwd_kernel(
     }
     if (k < k1) add(d0);
   }
+  add_parts<W, CPL, 9>(s_acc, local, part, lane, acc);
+  if (W > 1 && (!live || part > 0)) return;
   float* xo = x_out + n * 9 * C + c;
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
@@ -340,8 +357,22 @@ template <int CPL>
 static void launch_scatter_fwd(const int32_t* rptr, const int32_t* col, const float* Z0, const float* Z1,
                                const float* Z2, const float* wig, const float* env, const float* x_res, float* x_out,
                                int64_t N, hipStream_t st) {
-  hipLaunchKernelGGL(scatter_fwd_kernel<CPL>, dim3(cdiv(N, 4)), dim3(256), 0, st, rptr, col, Z0, Z1, Z2, wig, env,
-                     x_res, x_out, N);
+  with_waves<CPL>(node_waves(N), [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((scatter_fwd_kernel<CPL, W>), dim3(cdiv(N, 4 / W)), dim3(256), 0, st, rptr, col, Z0, Z1, Z2, wig,
+                       env, x_res, x_out, N);
+  });
+}
+
+template <int CPL>
+static void launch_init_scatter_fwd(const int32_t* rptr, const int32_t* col, const float* rad, const float* wig,
+                                    const float* env, const int64_t* Z, const int64_t* batch, const float* W_sphere,
+                                    const float* csd, float* x_out, int64_t N, hipStream_t st) {
+  with_waves<CPL>(node_waves(N), [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((init_scatter_fwd_kernel<CPL, W>), dim3(cdiv(N, 4 / W)), dim3(256), 0, st, rptr, col, rad, wig, env,
+                       Z, batch, W_sphere, csd, x_out, N);
+  });
 }
 
 template <int CPL>
@@ -415,16 +446,10 @@ extern "C" int fu_init_scatter_fwd(const int32_t* row_ptr, const int32_t* col_id
   if (!row_ptr || !Z || !batch || !W_sphere || !csd_emb || !x_out || (E > 0 && (!col_idx || !rad || !wigner || !env)))
     return set_error(FU_ERR_NULL, "fu_init_scatter_fwd: NULL argument");
   hipStream_t s = as_stream(stream);
-  const dim3 grid(cdiv(N, 4));
-  if (C == 64)
-    hipLaunchKernelGGL(init_scatter_fwd_kernel<1>, grid, dim3(256), 0, s, row_ptr, col_idx, rad, wigner, env, Z, batch,
-                       W_sphere, csd_emb, x_out, N);
+  if (C == 64) launch_init_scatter_fwd<1>(row_ptr, col_idx, rad, wigner, env, Z, batch, W_sphere, csd_emb, x_out, N, s);
   else if (C == 128)
-    hipLaunchKernelGGL(init_scatter_fwd_kernel<2>, grid, dim3(256), 0, s, row_ptr, col_idx, rad, wigner, env, Z, batch,
-                       W_sphere, csd_emb, x_out, N);
-  else
-    hipLaunchKernelGGL(init_scatter_fwd_kernel<4>, grid, dim3(256), 0, s, row_ptr, col_idx, rad, wigner, env, Z, batch,
-                       W_sphere, csd_emb, x_out, N);
+    launch_init_scatter_fwd<2>(row_ptr, col_idx, rad, wigner, env, Z, batch, W_sphere, csd_emb, x_out, N, s);
+  else launch_init_scatter_fwd<4>(row_ptr, col_idx, rad, wigner, env, Z, batch, W_sphere, csd_emb, x_out, N, s);
   return check_launch("fu_init_scatter_fwd");
 }
 
