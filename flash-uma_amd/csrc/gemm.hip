@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_k
   static_assert(SPLIT || !TALL, "tall tiles exist in the split mode only");
   static_assert(!GATHER || (SPLIT && !KTAIL && MODE == 1), "the gathered A operand feeds the split gate GEMM");
   static_assert(!F16 || (SPLIT && !GATHER), "the fp16 split is a split mode without the gathered loader");
-  static_assert(!WF || (F16 && TALL && !KTAIL), "pre-split weight fragments feed the tall fp16 tile without a K tail");
+  static_assert(!WF || (F16 && !KTAIL), "pre-split weight fragments feed the fp16 tiles without a K tail");
   constexpr int RB = TALL ? 4 : 2;          // 32-row blocks per wave
   constexpr int BM = 64 * RB;               // tile rows
   constexpr int PA = BM * GBK, PW = G_PLANE;  // bf16 per A plane, per W plane
@@ -995,15 +995,31 @@ static auto linear_kernel(int32_t K, int64_t M, int64_t bm = 0) {
          : mode == FU_MATMUL_SPLIT_F16 ? split_kernel<MODE, true>(K, tall) : split_kernel<MODE, false>(K, tall);
 }
 
-// With a pre-split weight (W2, fu_linear_weight_split of the same N x K weight): the tall fp16
-// tile reading its weight fragments from W2 (split-fp16 mode, tall tiles, K % 16 == 0);
-// otherwise W2 is not used.
+// With a pre-split weight (W2, fu_linear_weight_split of the same N x K weight; split-fp16 mode,
+// K % 16 == 0) the fp16 tiles read their weight fragments from W2 instead of staging and splitting
+// W in every workgroup.  Measured, us at 30,000 rows, W -> W2 on 128-row tiles: N 640, K 768 125 -> 117
+// (with the gate epilogue 143 -> 131), N 768, K 640 133 -> 122, N = K = 384 43 -> 40, the gate backward
+// 75 -> 72, K 1,536 with the LayerNorm backward 79 -> 66; at 6,000 rows 40 -> 35, 46 -> 41, 44 -> 41,
+// 23 -> 21, 41 -> 38.  Below that the launches take a few us more or less and the plain tiles stay.
+constexpr int64_t W2_MIN_ROWS = 4096;
 static bool use_w2(const void* W2, int32_t K, int64_t M) {
-  return W2 != nullptr && matmul_mode() == FU_MATMUL_SPLIT_F16 && linear_tile_rows(M) != GBM && K % GBK == 0;
+  return W2 != nullptr && matmul_mode() == FU_MATMUL_SPLIT_F16 && M >= W2_MIN_ROWS && K % GBK == 0;
+}
+// Tile rows of the W2 tiles: without the split of W a tall tile pays earlier where the epilogue is
+// short (MODE 0 and 1).  us, 128 -> 256 rows: 30,000 rows 122 -> 114, 117 -> 123, 131 -> 141, 40 -> 44
+// (the first four shapes above, N 768 first); 40,000 160 -> 145, 158 -> 152, 174 -> 177, 55 -> 49;
+// 50,000 198 -> 164, 194 -> 170, 205 -> 194, 68 -> 74; the gate backward 120 -> 149 at 50,000 and even
+// from 65,536 on.
+constexpr int64_t W2_TALL_MIN_ROWS = 36864;
+template <int MODE>
+static int64_t w2_tile_rows(const void* W2, int32_t K, int64_t M) {
+  return MODE <= 1 && use_w2(W2, K, M) && M >= W2_TALL_MIN_ROWS ? 2 * GBM : linear_tile_rows(M);
 }
 template <int MODE>
 static auto linear_kernel_w2(int32_t K, int64_t M, const void* W2) {
-  return use_w2(W2, K, M) ? linear_mfma_kernel<MODE, true, false, true, false, true, true> : linear_kernel<MODE>(K, M);
+  if (!use_w2(W2, K, M)) return linear_kernel<MODE>(K, M);
+  return w2_tile_rows<MODE>(W2, K, M) != GBM ? linear_mfma_kernel<MODE, true, false, true, false, true, true>
+                                             : linear_mfma_kernel<MODE, true, false, false, false, true, true>;
 }
 static int w2_check(const void* W2, const char* who) {
   return (W2 && !aligned16(W2)) ? set_error(FU_ERR_ALIGN, "%s: W2 must be 16-byte aligned", who) : FU_OK;
@@ -1031,7 +1047,7 @@ static int linear_launch(const float* A, int64_t lda, int64_t sA, const float* W
                          int64_t M, int32_t N, int32_t K, int32_t batch, hipStream_t stream, const char* who,
                          Resid rs = Resid{}, const void* W2 = nullptr) {
   const int n_tiles = (N + GBN - 1) / GBN;
-  const int64_t bm = linear_tile_rows(M);
+  const int64_t bm = w2_tile_rows<0>(W2, K, M);
   const int64_t m_tiles = (M + bm - 1) / bm;
   const int64_t total = m_tiles * n_tiles;
   if (total > 0x7fffffffLL) return set_error(FU_ERR_SHAPE, "%s: M too large", who);
@@ -1085,7 +1101,7 @@ extern "C" int fu_linear_gate(const float* A, int64_t lda, const float* W, int64
   if (ldz % 4 != 0 || !aligned16(Z) || (S && (lds % 4 != 0 || !aligned16(S))) || (bias && !aligned16(bias)))
     return set_error(FU_ERR_ALIGN, "%s: Z, S and bias must be 16-byte aligned with row strides multiples of 4", who);
   const int n_tiles = (N + GBN - 1) / GBN;
-  const int64_t bm = linear_tile_rows(M);
+  const int64_t bm = w2_tile_rows<1>(W2, K, M);
   const int64_t total = ((M + bm - 1) / bm) * n_tiles;
   if (total > 0x7fffffffLL) return set_error(FU_ERR_SHAPE, "%s: M too large", who);
   auto kern = linear_kernel_w2<1>(K, M, W2);
@@ -1148,7 +1164,7 @@ extern "C" int fu_linear_gate_bwd(const float* gZo, int64_t ldgz, const float* W
   if ((ldy0 | ldp1 | ldp2) % 4 != 0 || !aligned16(Y0) || !aligned16(P1) || !aligned16(P2))
     return set_error(FU_ERR_ALIGN, "%s: operands must be 16-byte aligned with row strides multiples of 4", who);
   const int n_tiles = (N + GBN - 1) / GBN;
-  const int64_t bm = linear_tile_rows(M);
+  const int64_t bm = w2_tile_rows<2>(W2, K, M);
   const int64_t total = ((M + bm - 1) / bm) * n_tiles;
   if (total > 0x7fffffffLL) return set_error(FU_ERR_SHAPE, "%s: M too large", who);
   auto kern = linear_kernel_w2<2>(K, M, W2);
@@ -1263,7 +1279,7 @@ extern "C" int fu_linear_dgrad_ln_silu_bwd(const float* A, int64_t lda, const fl
                         as_stream(stream));
     return check_launch(who);
   }
-  const int64_t bm = linear_tile_rows(M);
+  const int64_t bm = w2_tile_rows<5>(W2, K, M);
   const int64_t total = (M + bm - 1) / bm;
   if (total > 0x7fffffffLL) return set_error(FU_ERR_SHAPE, "%s: M too large", who);
   // the kernel addresses group 0 of its operands; the group's columns and statistics are

@@ -167,7 +167,7 @@ class Packed_eSCN_Layer(nn.Module):
     # factor keeps the four-product kernel (no pre-split copy).
     GAUSS_MAX_NORM_RATIO = 10.0
 
-    # the real m = 0 weights whose tall GEMMs read pre-split fragments (linear_weight_split), in
+    # the real m = 0 weights whose GEMMs read pre-split fragments (linear_weight_split), in
     # the order conv1_gate_conv2 takes them after the complex splits
     _REAL = ("W_conv1_m0", "W_conv1_m0_t", "W_conv2_m0", "W_conv2_m0_t")
 

@@ -12,7 +12,7 @@ from . import _lib
 def gemm(x: torch.Tensor, W: torch.Tensor, bias: torch.Tensor | None = None,
          out: torch.Tensor | None = None, W2: torch.Tensor | None = None) -> torch.Tensor:
     """out[M, N] = x[M, K] @ W[N, K]^T (+ bias).  x may be a row-strided view.  W2: W pre-split by
-    linear_weight_split, read instead of W where fu_linear can (split-fp16 mode, tall tiles)."""
+    linear_weight_split, read instead of W where fu_linear can (split-fp16 mode, 4,096 rows or more)."""
     if x.stride(-1) != 1:
         x = x.contiguous()
     M, K = x.shape

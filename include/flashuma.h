@@ -280,7 +280,7 @@ int fu_linear_dgrad_ln_silu_bwd(const float* A, int64_t lda, const float* W, int
  * multiples of 4 and A, W, Y 16-byte aligned.
  * W2 (here and in fu_linear_gate, fu_linear_gate_bwd, fu_linear_dgrad_ln_silu_bwd): NULL, or
  * the same weight pre-split by fu_linear_weight_split (16-byte aligned).  In matrix-core mode 2
- * with tall tiles (M >= 65,536) and K % 16 == 0 the kernel then loads its weight fragments from
+ * with M >= 4,096 and K % 16 == 0 the kernel then loads its weight fragments from
  * W2 straight into registers (exact column scales and window flags from W2) instead of staging
  * and splitting W; otherwise W2 is not read.  No reference counterpart (an argument of this
  * build's kernels). */

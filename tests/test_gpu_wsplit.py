@@ -199,3 +199,26 @@ def test_radial_bank_backward_with_weight_fragments(cuda, monkeypatch):
             cots = [torch.randn(o.shape, device=cuda, generator=g) for o in outs]
         (res[tag],) = torch.autograd.grad(outs, [gg], cots)
     assert _normwise(res["w2"], res["plain"]) <= 2e-6, _normwise(res["w2"], res["plain"])
+
+
+@pytest.mark.parametrize("M,N,K", [(4095, 64, 384), (4096, 128, 1536), (4097, 200, 64), (4500, 640, 768), (36863, 96, 80),
+                                   (36864, 96, 80), (36865, 320, 96)])
+def test_weight_fragments_by_rows(cuda, M, N, K):
+    """Both sides of the lines of W2 (4,096 rows) and its tall tiles (36,864 rows), ragged last row and
+    column tiles, K of 4, 5 and more chunks, rows of zeros: against float64, next to the plain tiles."""
+    _lib, linear = _ops()
+    g = torch.Generator().manual_seed(M + N + K)
+    x, W, b = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5, torch.randn(N, generator=g)
+    x[5::31] = 0.0
+    x[7::64, :16] = 0.0
+    x, W, b = x.to(cuda), W.to(cuda), b.to(cuda)
+    W2 = linear.linear_weight_split(W)
+    ref = x.double() @ W.double().T + b.double()
+    y, plain = linear.gemm(x, W, b, W2=W2), linear.gemm(x, W, b)
+    err = [((v.double() - ref).norm() / ref.norm()).item() for v in (y, plain)]
+    mx = [((v.double() - ref).abs().max() / ref.abs().max()).item() for v in (y, plain)]
+    # 22-bit operands, fp32 accumulation over K: as the plain tiles
+    assert err[0] < 1e-6 and err[0] <= 1.1 * err[1] and mx[0] <= 1.5 * mx[1], (err, mx)
+    assert torch.equal(y[5::31], b.expand_as(y[5::31]))
+    if M < 4096:
+        assert torch.equal(y, plain)
