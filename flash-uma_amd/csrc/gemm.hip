@@ -948,6 +948,24 @@ __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_k
   }
 }
 
+void launch_linear_rows16(const float* A, int64_t lda, int64_t sA, const float* W, int64_t ldw, int64_t sW,
+                          const float* bias, int64_t sBias, int32_t bias_batches, const float* R, int64_t ldr,
+                          int64_t sR, float* Y, int64_t ldy, int64_t sY, int64_t M, int32_t N, int32_t K,
+                          int32_t batch, hipStream_t s);
+// fu_linear_batched on the 16-row tiles of gemm_rows16.hip: while their workgroups (16 rows, one batch
+// entry, 128 columns) are all on the chip at once, two a CU; past that the repeated weight reads and the
+// fp32 rate cost more than the 128-row tiles' idle CUs.  Measured, us, 128 / 16 rows: nine products of
+// 128 x 128 10.9 / 6.2 at 54 rows (36 workgroups), 11.4 / 8.4 at 500 (288), 11.5 / 11.0 at 999 (567), 11.7 /
+// 16.8 at 2,000; 25 of them 11.5 / 8.7 at 250 (400), 11.6 / 14.2 at 500 (800); nine of 256 x 256 15.4 / 14.2
+// at 250 (288), 15.6 / 19.1 at 500 (576); one of 256 x 128 12.2 / 6.2 at 54, 13.1 / 8.7 at 4,000 (500).
+// Batches past 512 rows are the radial MLP's hidden layers, whose products fu_linear_ln_silu writes
+// too, from 128-row tiles: the two stay the same bit for bit.
+constexpr int64_t ROWS16_MAX_GROUPS = 512, ROWS16_MAX_BATCHED_ROWS = 512;
+static bool use_rows16(int64_t M, int32_t N, int32_t K, int32_t batch) {
+  return N % 16 == 0 && K % 32 == 0 && (batch == 1 || M <= ROWS16_MAX_BATCHED_ROWS) &&
+         M <= 16 * ROWS16_MAX_GROUPS && ((M + 15) / 16) * batch * ((N + 127) / 128) <= ROWS16_MAX_GROUPS;
+}
+
 void launch_short_ln_bwd(const float* A, int64_t lda, const void* W2, float* g_x, int64_t ldgx, int64_t M, int32_t K,
                          const float* x, int64_t ldx, const float* gamma, const float* beta, const float* mean,
                          const float* rstd, int32_t G, hipStream_t st);   // gemm_short.hip
@@ -1080,6 +1098,11 @@ extern "C" int fu_linear_batched(const float* A, int64_t lda, int64_t stride_a, 
   if (R && ((ldr | stride_r) % 4 != 0 || ldr < N || stride_r < 0 || !aligned16(R)))
     return set_error(FU_ERR_ALIGN, "fu_linear_batched: R must be 16-byte aligned with ldr >= N, strides multiples of 4");
   if (M == 0) return FU_OK;
+  if (use_rows16(M, N, K, batch)) {
+    launch_linear_rows16(A, lda, stride_a, W, ldw, stride_w, bias, stride_bias, bias_batches, R, ldr, stride_r, Y, ldy,
+                         stride_y, M, N, K, batch, as_stream(stream));
+    return check_launch("fu_linear_batched");
+  }
   return linear_launch(A, lda, stride_a, W, ldw, stride_w, bias, stride_bias, bias_batches, Y, ldy, stride_y, M, N, K,
                        batch, as_stream(stream), "fu_linear_batched", Resid{R, ldr, stride_r});
 }

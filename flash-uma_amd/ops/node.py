@@ -84,6 +84,17 @@ def _so3_apply(x: torch.Tensor, Wk: torch.Tensor, bias: torch.Tensor | None,
     return y
 
 
+def _scalar_gemm(x: torch.Tensor, W: torch.Tensor, b: torch.Tensor | None, add_to: torch.Tensor | None = None):
+    """x[:, 0] @ W^T (+ b) of x (N, K, Cin) or (N, Cin), or, with add_to (N, K, Cout), add_to[:, 0] += it in
+    place (the residual of the GEMM's epilogue)."""
+    N, O, I = x.shape[0], W.shape[0], W.shape[1]
+    y = torch.empty(N, O, device=x.device, dtype=torch.float32) if add_to is None else add_to
+    _lib.call("fu_linear_batched", x.data_ptr(), x.stride(0), 0, W.data_ptr(), W.stride(0), 0, _lib.ptr(b), 0, 1,
+              None if add_to is None else y.data_ptr(), y.stride(0), 0, y.data_ptr(), y.stride(0), 0, N, O, I, 1,
+              _lib.stream_ptr(x.device))
+    return y
+
+
 class So3Linear(torch.autograd.Function):
     """x (N, K, Cin) -> (N, K, Cout) with a weight per coefficient k: W_k (Cout, Cin)
     (the weight of k's degree), bias on k = 0.  Wt_k = W_k^T for the input gradient."""
@@ -133,20 +144,18 @@ class ScalarGemmSo3(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, W, b, Wt, Wk, Wtk, bias):
-        from .linear import gemm
         x = _lib.require(x, torch.float32, "x")
-        pre = gemm(x[:, 0, :], W, b)
+        pre = _scalar_gemm(x, W, b)
         h = _so3_apply(x, Wk, bias)
         ctx.save_for_backward(Wt, Wtk)
         return pre, h
 
     @staticmethod
     def backward(ctx, g_pre, g_h):
-        from .linear import gemm
         Wt, Wtk = ctx.saved_tensors
         g_x = _so3_apply(g_h.contiguous(), Wtk, None)
         if g_pre is not None:
-            g_x[:, 0, :] += gemm(g_pre.contiguous(), Wt)
+            _scalar_gemm(g_pre.contiguous(), Wt, None, g_x)
         return g_x, None, None, None, None, None, None
 
 

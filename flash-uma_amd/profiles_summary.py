@@ -37,6 +37,7 @@ KERNEL_ENTRY = {
     "radial_gather_kernel": "fu_radial_gather_fwd", "radial_gather_lmax_kernel": "fu_radial_gather_fwd_lmax",
     "short_kernel": "fu_so2_pair_fwd/bwd, fu_linear_short", "short_ln_bwd_kernel": "fu_linear_dgrad_ln_silu_bwd",
     "rms_norm_fwd_kernel": "fu_rms_norm_sh_fwd", "rms_norm_bwd_kernel": "fu_rms_norm_sh_bwd",
+    "linear_rows16_kernel": "fu_linear_batched",
     "gate_fwd_kernel": "fu_gate_act_fwd", "gate_bwd_kernel": "fu_gate_act_bwd",
     "gather_rows_kernel": "fu_gather_rows", "scatter_rows_kernel": "fu_scatter_rows",
     "edge_shifts_kernel": "fu_edge_shifts", "outer_sum3_stage1": "fu_outer_sum3", "outer_sum3_stage2": "fu_outer_sum3",

@@ -146,3 +146,29 @@ def test_dgrad_ln_silu_short(cuda, M, K, group):
     (ref,) = torch.autograd.grad(y, v, A.double() @ W.double().T)
     e, t = _err(outs, [ref.cpu()] * 2)
     assert e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
+
+
+@pytest.mark.parametrize("M,N,K,batch", [(1, 16, 32, 3), (15, 128, 128, 9), (16, 144, 96, 1), (17, 256, 160, 2),
+                                         (54, 128, 128, 25), (512, 64, 64, 5), (513, 64, 64, 5), (2049, 128, 384, 1),
+                                         (4096, 256, 128, 1), (8200, 128, 32, 1)])
+def test_linear_batched_few_rows(cuda, M, N, K, batch):
+    """fu_linear_batched on its 16-row tiles and just past them: interleaved batches (row stride over all of
+    them), a bias on the first batches only, and a residual that is the output itself, against float64
+    and a plain fp32 product of torch; the columns between the batches keep their contents."""
+    from ops import _lib
+    g = torch.Generator().manual_seed(M + N + K)
+    r = lambda *s: torch.randn(*s, generator=g)
+    A, W, b, R = r(M, batch, K + 4), r(batch, N, K) / K ** 0.5, r(batch, N), r(M, batch, N + 4)
+    nb = min(2, batch)
+    bias = torch.cat([b[:nb], torch.zeros(batch - nb, N)])
+    x64 = A[..., :K].double()
+    ref = torch.stack([x64[:, i] @ W[i].double().T for i in range(batch)], 1) + bias.double() + R[..., :N].double()
+    Ad, Wd, bd, Y = (t.to(cuda) for t in (A, W, b, R))
+    _lib.call("fu_linear_batched", Ad.data_ptr(), batch * (K + 4), K + 4, Wd.data_ptr(), K, N * K, bd.data_ptr(), N, nb,
+              Y.data_ptr(), batch * (N + 4), N + 4, Y.data_ptr(), batch * (N + 4), N + 4, M, N, K, batch,
+              _lib.stream_ptr(cuda))
+    plain = torch.stack([A[:, i, :K] @ W[i].T for i in range(batch)], 1) + bias + R[..., :N]
+    e, t = _err([Y[..., :N], plain], [ref, ref])
+    # fp32 products in sums of K / 4 terms, or 22-bit operands past the rule
+    assert e <= 1e-6 and e <= 2.0 * t + 1e-7, (e, t)
+    assert torch.equal(Y[..., N:].cpu(), R[..., N:])
