@@ -13,10 +13,14 @@
 // per atom; atoms are then sorted by bin (fu_sort_pairs_i64) and bin ranges found
 // (fu_csr_row_ptr).  Bins are at least cutoff + 1e-3 wide, so with `reach` bins searched
 // per side every neighbour is visited exactly once per periodic image.  (2) fu_nlist_search:
-// one wave per receiver walks the neighbouring bins, tests 64 candidates at a time, appends
-// hits to an LDS list (ballot + prefix count), then ranks the list by the ordering key
-// (each entry's rank = number of smaller keys; keys are unique) and writes the first
-// max_neighbors.  (3) fu_nlist_scan: exclusive scan of the per-receiver counts.
+// one wave per receiver reads the ranges of the neighbouring bins, one a lane, tests the atoms in them
+// 64 at a time across bins, appends hits to an LDS list (ballot + prefix count), then ranks the list
+// by the ordering key (each entry's rank = number of smaller keys; keys are unique) and writes the
+// first max_neighbors.  Bound by latency: bin by bin, a receiver of 27 bins of about ten atoms waited
+// for three dependent loads at each, 233 us for 20,000 atoms; 64 candidates at a time 137, and 107
+// with an entry of the list in one LDS read and no branch where distances are equal.
+// (3) fu_nlist_scan: exclusive scan of the per-receiver counts (20,000 of them: 8 us, 28 by one
+// workgroup).
 // (4) fu_nlist_emit: edge_index (2, E) int64 and cell_offsets (E, 3) float32.
 #include "fu_common.h"
 
@@ -76,8 +80,13 @@ __global__ __launch_bounds__(256) void nlist_search_kernel(
     const int32_t* __restrict__ wrap, const int64_t* __restrict__ bin_key, NLGeom g, int64_t N, int32_t K,
     int32_t* __restrict__ out_sender, int32_t* __restrict__ out_off, int32_t* __restrict__ count,
     int32_t* __restrict__ nout) {
-  __shared__ double s_d2[4][NL_CAP];
-  __shared__ uint64_t s_key[4][NL_CAP];  // (i << 24) | (o0 + 128) << 16 | (o1 + 128) << 8 | (o2 + 128)
+  // hits: d^2 and (i << 24) | (o0 + 128) << 16 | (o1 + 128) << 8 | (o2 + 128), side by side so that an
+  // entry is one LDS read
+  struct __attribute__((aligned(16))) Hit {
+    double d2;
+    uint64_t key;
+  };
+  __shared__ Hit s_hit[4][NL_CAP];
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int64_t j = (int64_t)blockIdx.x * 4 + w;
@@ -88,62 +97,107 @@ __global__ __launch_bounds__(256) void nlist_search_kernel(
     const int wj[3] = {wrap[3 * j], wrap[3 * j + 1], wrap[3 * j + 2]};
     const int64_t kj = bin_key[j];
     const int bj[3] = {(int)(kj / ((int64_t)g.nb[1] * g.nb[2])), (int)((kj / g.nb[2]) % g.nb[1]), (int)(kj % g.nb[2])};
-    for (int dx = -g.reach[0]; dx <= g.reach[0]; ++dx)
-      for (int dy = -g.reach[1]; dy <= g.reach[1]; ++dy)
-        for (int dz = -g.reach[2]; dz <= g.reach[2]; ++dz) {
-          const int u[3] = {bj[0] + dx, bj[1] + dy, bj[2] + dz};
-          int nbn[3], kk[3];
+    const int ny = 2 * g.reach[1] + 1, nz = 2 * g.reach[2] + 1, total = (2 * g.reach[0] + 1) * ny * nz;
+    const int per = N < (1 << 25) ? 64 : 1;   // bins a time: their candidates are counted in 32 bits
+    for (int q0 = 0; q0 < total; q0 += per) {
+      // a bin per lane: its image, its first atom and, summed over the lanes before, its first
+      // candidate; the candidates of the 64 bins are then taken 64 at a time whatever bin they are
+      // in, so one receiver waits for its loads about every 64 candidates and not at every bin
+      const int q = q0 + lane;
+      int kk[3] = {0, 0, 0}, lo = 0, len = 0;
+      if (lane < per && q < total) {
+        const int u[3] = {bj[0] + q / (ny * nz) - g.reach[0], bj[1] + (q / nz) % ny - g.reach[1], bj[2] + q % nz - g.reach[2]};
+        int nbn[3];
 #pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            kk[a] = floor_div(u[a], g.nb[a]);
-            nbn[a] = u[a] - kk[a] * g.nb[a];
-          }
-          const int64_t bin = ((int64_t)nbn[0] * g.nb[1] + nbn[1]) * g.nb[2] + nbn[2];
-          const int32_t lo = bin_ptr[bin], hi = bin_ptr[bin + 1];
-          for (int32_t t = lo; t < hi; t += 64) {
-            const int32_t idx = t + lane;
-            bool hit = false;
-            double d2 = 0.0;
-            uint64_t key = 0;
-            if (idx < hi) {
-              const int64_t i = sorted_atoms[idx];
-              int o[3];
-#pragma unroll
-              for (int a = 0; a < 3; ++a) o[a] = g.pbc[a] ? kk[a] - wrap[3 * i + a] + wj[a] : 0;
-              const bool self = (i == j) && o[0] == 0 && o[1] == 0 && o[2] == 0;
-              const double pi[3] = {(double)pos[3 * i], (double)pos[3 * i + 1], (double)pos[3 * i + 2]};
-              d2 = pair_d2(pi, pj, o, g.cell);
-              hit = !self && d2 < g.cut2;
-              key = ((uint64_t)i << 24) | ((uint64_t)(o[0] + 128) << 16) | ((uint64_t)(o[1] + 128) << 8) |
-                    (uint64_t)(o[2] + 128);
-            }
-            const uint64_t mask = __ballot(hit);
-            const int slot = cnt + __popcll(mask & ((1ull << lane) - 1ull));
-            if (hit && slot < NL_CAP) {
-              s_d2[w][slot] = d2;
-              s_key[w][slot] = key;
-            }
-            cnt += __popcll(mask);
-          }
+        for (int a = 0; a < 3; ++a) {
+          kk[a] = floor_div(u[a], g.nb[a]);
+          nbn[a] = u[a] - kk[a] * g.nb[a];
         }
+        const int64_t bin = ((int64_t)nbn[0] * g.nb[1] + nbn[1]) * g.nb[2] + nbn[2];
+        lo = bin_ptr[bin];
+        len = bin_ptr[bin + 1] - lo;
+      }
+      int first = len;
+#pragma unroll
+      for (int s = 1; s < 64; s <<= 1) {
+        const int v = __shfl_up(first, s, 64);
+        if (lane >= s) first += v;
+      }
+      const int cands = __shfl(first, 63, 64);
+      first -= len;
+      // candidate c: the last bin whose first candidate is at or before c (empty bins share theirs with
+      // the next one, which is later)
+      auto bin_of = [&](int64_t c) {
+        int p = 0;
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1)
+          if (__shfl(first, p + s, 64) <= c) p += s;
+        return p;
+      };
+      auto atom_of = [&](int64_t c, int p) {
+        const int64_t at = __shfl(lo, p, 64) + c - __shfl(first, p, 64);
+        return c < cands ? sorted_atoms[at] : (int64_t)0;
+      };
+      int p = bin_of(lane);
+      int64_t i = atom_of(lane, p);
+      for (int64_t c0 = 0; c0 < cands; c0 += 64) {
+        const int pn = bin_of(c0 + 64 + lane);
+        const int64_t in = atom_of(c0 + 64 + lane, pn);   // the next candidates' atoms, one step ahead
+        const int kc[3] = {__shfl(kk[0], p, 64), __shfl(kk[1], p, 64), __shfl(kk[2], p, 64)};
+        bool hit = false;
+        double d2 = 0.0;
+        uint64_t key = 0;
+        if (c0 + lane < cands) {
+          int o[3];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) o[a] = g.pbc[a] ? kc[a] - wrap[3 * i + a] + wj[a] : 0;
+          const bool self = (i == j) && o[0] == 0 && o[1] == 0 && o[2] == 0;
+          const double pi[3] = {(double)pos[3 * i], (double)pos[3 * i + 1], (double)pos[3 * i + 2]};
+          d2 = pair_d2(pi, pj, o, g.cell);
+          hit = !self && d2 < g.cut2;
+          key = ((uint64_t)i << 24) | ((uint64_t)(o[0] + 128) << 16) | ((uint64_t)(o[1] + 128) << 8) |
+                (uint64_t)(o[2] + 128);
+        }
+        const uint64_t mask = __ballot(hit);
+        const int slot = cnt + __popcll(mask & ((1ull << lane) - 1ull));
+        if (hit && slot < NL_CAP) s_hit[w][slot] = Hit{d2, key};
+        cnt += __popcll(mask);
+        p = pn;
+        i = in;
+      }
+    }
   }
   __syncthreads();
   if (!active) return;
   const int n = cnt < NL_CAP ? cnt : NL_CAP;
-  for (int e = lane; e < n; e += 64) {
-    const double de = s_d2[w][e];
-    const uint64_t ke = s_key[w][e];
-    int rank = 0;
-    for (int f = 0; f < n; ++f) {
-      const double df = s_d2[w][f];
-      rank += (df < de || (df == de && s_key[w][f] < ke)) ? 1 : 0;
+  // two entries per lane and walk of the list
+  for (int e0 = 0; e0 < n; e0 += 128) {
+    double de[2];
+    uint64_t ke[2];
+    int rank[2] = {0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int e = e0 + 64 * h + lane;
+      const Hit x = s_hit[w][e < n ? e : 0];
+      de[h] = x.d2;
+      ke[h] = x.key;
     }
-    if (rank < K) {
-      const int64_t slot = j * K + rank;
-      out_sender[slot] = (int32_t)(ke >> 24);
-      out_off[3 * slot + 0] = (int)((ke >> 16) & 0xff) - 128;
-      out_off[3 * slot + 1] = (int)((ke >> 8) & 0xff) - 128;
-      out_off[3 * slot + 2] = (int)(ke & 0xff) - 128;
+    // no branch on equal distances: an entry always meets itself, and lattices are full of them
+#pragma unroll 4
+    for (int f = 0; f < n; ++f) {
+      const Hit x = s_hit[w][f];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) rank[h] += (int)(x.d2 < de[h]) | ((int)(x.d2 == de[h]) & (int)(x.key < ke[h]));
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      if (e0 + 64 * h + lane < n && rank[h] < K) {
+        const int64_t slot = j * K + rank[h];
+        out_sender[slot] = (int32_t)(ke[h] >> 24);
+        out_off[3 * slot + 0] = (int)((ke[h] >> 16) & 0xff) - 128;
+        out_off[3 * slot + 1] = (int)((ke[h] >> 8) & 0xff) - 128;
+        out_off[3 * slot + 2] = (int)(ke[h] & 0xff) - 128;
+      }
     }
   }
   if (lane == 0) {
@@ -152,29 +206,66 @@ __global__ __launch_bounds__(256) void nlist_search_kernel(
   }
 }
 
-// Exclusive scan of nout into row_ptr (N + 1 entries, row_ptr[N] = E) by one workgroup.
+// Exclusive scan of nout into row_ptr (N + 1 entries, row_ptr[N] = E).  Up to 256 workgroups, each with
+// a span of whole 1,024s: a workgroup sums the counts before its span (coalesced, from the L2)
+// instead of waiting for the workgroups before it, then scans its span 1,024 at a time.
 __global__ __launch_bounds__(1024) void nlist_scan_kernel(const int32_t* __restrict__ nout, int64_t* __restrict__ row_ptr,
-                                                          int64_t N) {
-  __shared__ int64_t s[1024];
-  const int t = threadIdx.x;
-  const int64_t chunk = (N + 1023) / 1024;
-  const int64_t b = t * chunk, e = b + chunk < N ? b + chunk : N;
-  int64_t sum = 0;
-  for (int64_t k = b; k < e; ++k) sum += nout[k];
-  s[t] = sum;
+                                                          int64_t N, int64_t span) {
+  __shared__ int64_t s_base[16], s_sum[2][16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t b0 = (int64_t)blockIdx.x * span, b1 = b0 + span < N ? b0 + span : N;
+  int64_t base = 0;
+  for (int64_t m = t; m < b0; m += 1024) base += nout[m];
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) base += __shfl_xor(base, s, 64);
+  if (lane == 0) s_base[wave] = base;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int64_t v = t >= off ? s[t - off] : 0;
-    __syncthreads();
-    s[t] += v;
-    __syncthreads();
+  int64_t before = 0;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) before += s_base[v];
+  int buf = 0;
+  for (int64_t k0 = b0; k0 < b1; k0 += 1024, buf ^= 1) {
+    const int64_t k = k0 + t, own = k < b1 ? nout[k] : 0;
+    int64_t run = own;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int64_t v = __shfl_up(run, s, 64);
+      if (lane >= s) run += v;
+    }
+    if (lane == 63) s_sum[buf][wave] = run;
+    __syncthreads();   // the other buffer's readers are past the previous tile's barrier
+    int64_t prior = 0, all = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      prior += v < wave ? s_sum[buf][v] : 0;
+      all += s_sum[buf][v];
+    }
+    if (k < b1) row_ptr[k] = before + prior + run - own;
+    before += all;
   }
-  int64_t run = t ? s[t - 1] : 0;
-  for (int64_t k = b; k < e; ++k) {
-    row_ptr[k] = run;
-    run += nout[k];
+  if (b1 == N && t == 0) row_ptr[N] = before;
+}
+
+// limits[0], limits[1] (zeroed by the caller) = the largest |wrap| and the largest count
+__global__ __launch_bounds__(256) void nlist_limits_kernel(const int32_t* __restrict__ wrap,
+                                                           const int32_t* __restrict__ count, int64_t N,
+                                                           int64_t* __restrict__ limits) {
+  int m[2] = {0, 0};
+  for (int64_t a = (int64_t)blockIdx.x * 256 + threadIdx.x; a < 3 * N; a += (int64_t)gridDim.x * 256) {
+    const int v = wrap[a], u = v < 0 ? (int)(0u - (unsigned)v) : v;
+    m[0] = u > m[0] ? u : m[0];
+    if (a < N) m[1] = count[a] > m[1] ? count[a] : m[1];
   }
-  if (t == 1023) row_ptr[N] = s[1023];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int v = __shfl_xor(m[h], s, 64);
+      m[h] = v > m[h] ? v : m[h];
+    }
+    if ((threadIdx.x & 63) == 0 && m[h] > 0)
+      atomicMax(reinterpret_cast<unsigned long long*>(limits + h), (unsigned long long)m[h]);
+  }
 }
 
 __global__ __launch_bounds__(256) void nlist_emit_kernel(const int32_t* __restrict__ sender,
@@ -264,8 +355,19 @@ extern "C" int fu_nlist_search(const float* pos, const int64_t* sorted_atoms, co
 extern "C" int fu_nlist_scan(const int32_t* nout, int64_t* row_ptr, int64_t N, void* stream) {
   if (N < 0) return set_error(FU_ERR_SHAPE, "fu_nlist_scan: bad shape");
   if (!row_ptr || (N > 0 && !nout)) return set_error(FU_ERR_NULL, "fu_nlist_scan: NULL argument");
-  hipLaunchKernelGGL(nlist_scan_kernel, dim3(1), dim3(1024), 0, as_stream(stream), nout, row_ptr, N);
+  const int64_t span = 1024 * std::max<int64_t>(1, (N + 256 * 1024 - 1) / (256 * 1024));
+  hipLaunchKernelGGL(nlist_scan_kernel, dim3(std::max(1u, cdiv(N, span))), dim3(1024), 0, as_stream(stream), nout, row_ptr,
+                     N, span);
   return check_launch("fu_nlist_scan");
+}
+
+extern "C" int fu_nlist_limits(const int32_t* wrap, const int32_t* count, int64_t N, int64_t* limits, void* stream) {
+  if (N < 0) return set_error(FU_ERR_SHAPE, "fu_nlist_limits: bad shape");
+  if (N == 0) return FU_OK;
+  if (!wrap || !count || !limits) return set_error(FU_ERR_NULL, "fu_nlist_limits: NULL argument");
+  hipLaunchKernelGGL(nlist_limits_kernel, dim3((unsigned)std::min<int64_t>(cdiv(3 * N, 256), 256)), dim3(256), 0,
+                     as_stream(stream), wrap, count, N, limits);
+  return check_launch("fu_nlist_limits");
 }
 
 extern "C" int fu_nlist_emit(const int32_t* sender, const int32_t* off, const int32_t* nout, const int64_t* row_ptr,

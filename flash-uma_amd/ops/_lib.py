@@ -90,6 +90,7 @@ SIGNATURES: dict[str, list] = {
     "fu_nlist_bin": [P, I64, P, P, P, P, P, P, P, P],
     "fu_nlist_search": [P, P, P, P, P, I64, P, P, P, P, P, ctypes.c_double, I32, P, P, P, P, P],
     "fu_nlist_scan": [P, P, I64, P],
+    "fu_nlist_limits": [P, P, I64, P, P],
     "fu_nlist_emit": [P, P, P, P, I64, I32, P, P, I64, P],
     "fu_wigner_ext_width": [I32],
     "fu_wigner_ext_fwd": [P, P, I64, I32, P],

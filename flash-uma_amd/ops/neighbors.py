@@ -61,8 +61,6 @@ def radius_graph(pos: torch.Tensor, cell, pbc, cutoff: float, max_neighbors: int
     wrap = torch.empty(N, 3, dtype=torch.int32, device=dev)
     _lib.call("fu_nlist_bin", pos.data_ptr(), N, ptr(cell_h), ptr(inv_h), ptr(nb_h), ptr(reach_h), ptr(pbc_h),
               key.data_ptr(), wrap.data_ptr(), st)
-    if int(wrap.abs().max().item()) > _MAX_WRAP:
-        raise _lib.FlashUMAError("radius_graph: positions lie too far outside the cell; wrap them first")
     nbins = int(np.prod(nb_h))
     bin_ptr, atoms, sorted_keys = csr_from_keys(key, nbins)
     K = int(max_neighbors)
@@ -73,10 +71,15 @@ def radius_graph(pos: torch.Tensor, cell, pbc, cutoff: float, max_neighbors: int
     _lib.call("fu_nlist_search", pos.data_ptr(), atoms.data_ptr(), bin_ptr.data_ptr(), wrap.data_ptr(),
               key.data_ptr(), N, ptr(cell_h), ptr(inv_h), ptr(nb_h), ptr(reach_h), ptr(pbc_h), float(cutoff), K,
               sender.data_ptr(), off.data_ptr(), count.data_ptr(), nout.data_ptr(), st)
-    row_ptr = torch.empty(N + 1, dtype=torch.int64, device=dev)
+    # row_ptr and, after it, the largest |wrap| and count: read back with E in one copy (a graph whose
+    # wraps are out of range holds meaningless offsets but only indices below 2^31 are formed from them)
+    row_ptr = torch.zeros(N + 3, dtype=torch.int64, device=dev)
     _lib.call("fu_nlist_scan", nout.data_ptr(), row_ptr.data_ptr(), N, st)
-    E = int(row_ptr[N].item())
-    if int(count.max().item()) > NL_CAP:
+    _lib.call("fu_nlist_limits", wrap.data_ptr(), count.data_ptr(), N, row_ptr[N + 1:].data_ptr(), st)
+    E, max_wrap, max_count = row_ptr[N:].tolist()
+    if max_wrap > _MAX_WRAP:
+        raise _lib.FlashUMAError("radius_graph: positions lie too far outside the cell; wrap them first")
+    if max_count > NL_CAP:
         raise _lib.FlashUMAError(f"radius_graph: more than {NL_CAP} atoms within the cutoff of one receiver")
     edge_index = torch.empty(2, E, dtype=torch.int64, device=dev)
     cell_offsets = torch.empty(E, 3, dtype=torch.float32, device=dev)

@@ -45,7 +45,7 @@ KERNEL_ENTRY = {
     "morton_keys_kernel": "fu_morton_keys", "invert_perm_kernel": "fu_invert_perm", "take_i64_kernel": "fu_take_i64",
     "csr_row_ptr_kernel": "fu_csr_row_ptr", "narrow_kernel": "fu_narrow_i64_i32",
     "nlist_bin_kernel": "fu_nlist_bin", "nlist_search_kernel": "fu_nlist_search", "nlist_scan_kernel": "fu_nlist_scan",
-    "nlist_emit_kernel": "fu_nlist_emit",
+    "nlist_emit_kernel": "fu_nlist_emit", "nlist_limits_kernel": "fu_nlist_limits",
     "wigner_ext_fwd_kernel": "fu_wigner_ext_fwd", "wigner_ext_bwd_kernel": "fu_wigner_ext_bwd",
     "gather_fwd_lmax_kernel": "fu_gather_fwd_lmax", "gather_fwd_node_lmax_kernel": "fu_gather_fwd_lmax",
     "gather_bwd_lmax_kernel": "fu_gather_bwd_lmax",

@@ -611,6 +611,10 @@ int fu_nlist_search(const float* pos, const int64_t* sorted_atoms, const int32_t
 /* row_ptr (N + 1 int64) = exclusive scan of nout; row_ptr[N] = E. */
 int fu_nlist_scan(const int32_t* nout, int64_t* row_ptr, int64_t N, void* stream);
 
+/* limits (2 int64, zeroed by the caller) = the largest |wrap| of any axis and the largest count: the two
+ * conditions under which the graph is not valid, for the caller to read with row_ptr[N]. */
+int fu_nlist_limits(const int32_t* wrap, const int32_t* count, int64_t N, int64_t* limits, void* stream);
+
 /* edge_index (2 x E int64: senders, then receivers) and cell_offsets (E x 3 float32). */
 int fu_nlist_emit(const int32_t* sender, const int32_t* off, const int32_t* nout, const int64_t* row_ptr,
                   int64_t N, int32_t max_neighbors, int64_t* edge_index, float* cell_offsets, int64_t E,

@@ -158,3 +158,41 @@ def test_neighbor_list_skin_reuse(cuda):
     cell2 = np.asarray(s.cell, np.float64) * 1.001
     nl(pos0 + 0.31 * torch.tensor([1.0, 0.0, 0.0], device=cuda), cell2, s.pbc)
     assert nl.builds == 3
+
+
+@pytest.mark.parametrize("N", [0, 1, 1023, 1024, 1025, 262144, 262145, 600001])
+def test_nlist_scan_and_limits(cuda, N):
+    """The scan over one workgroup, several, and spans of several tiles, and the limits' maxima, against
+    numpy (whole numbers: exact)."""
+    import numpy as np
+    from ops import _lib
+    rng = np.random.default_rng(N)
+    nout, wrap = rng.integers(0, 64, N, dtype=np.int32), rng.integers(-61, 40, (N, 3), dtype=np.int32)
+    count = rng.integers(0, 700, N, dtype=np.int32)
+    d = [torch.from_numpy(a).to(cuda) for a in (nout, wrap, count)]
+    row = torch.zeros(N + 3, dtype=torch.int64, device=cuda)
+    st = _lib.stream_ptr(cuda)
+    _lib.call("fu_nlist_scan", d[0].data_ptr(), row.data_ptr(), N, st)
+    _lib.call("fu_nlist_limits", d[1].data_ptr(), d[2].data_ptr(), N, row[N + 1:].data_ptr(), st)
+    got = row.cpu().numpy()
+    assert (got[:N + 1] == np.concatenate([[0], np.cumsum(nout.astype(np.int64))])).all()
+    if N:
+        assert got[N + 1] == np.abs(wrap).max() and got[N + 2] == count.max()
+
+
+@pytest.mark.parametrize("n,a,pbc", [(1, 2.3, (1, 1, 1)), (2, 1.9, (1, 1, 0)), (3, 2.6, (1, 1, 1)), (5, 40.0, (0, 0, 0)),
+                                     (70, 14.0, (1, 0, 1)), (400, 13.0, (1, 1, 1))])
+def test_radius_graph_many_bins(cuda, n, a, pbc):
+    """More than 64 bins around a receiver (images of a small cell), one bin of all atoms, empty bins:
+    the host builder's graph, edge for edge, with equal distances (a lattice) among them."""
+    import numpy as np
+    import systems
+    from ops.neighbors import radius_graph
+    rng = np.random.default_rng(n)
+    cell = np.diag([a, a, a * 1.1]).astype(np.float32)
+    pos = (rng.integers(0, 8, (n, 3)) / 8 * a + (0.01 * rng.random((n, 3)) if n > 5 else 0)).astype(np.float32)
+    pos = np.unique(pos, axis=0)
+    pbc = np.array(pbc, dtype=bool)
+    ei, off = systems.neighbor_list(pos, cell, pbc, 6.0, 30)
+    gi, go = radius_graph(torch.from_numpy(pos).to(cuda), cell, pbc, 6.0, 30)
+    assert np.array_equal(gi.cpu().numpy(), ei) and np.array_equal(go.cpu().numpy(), off)
