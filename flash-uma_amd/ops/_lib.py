@@ -80,6 +80,8 @@ SIGNATURES: dict[str, list] = {
     "fu_gather_rows": [P, P, P, I64, I32, P],
     "fu_scatter_rows": [P, P, P, I64, I32, P],
     "fu_edge_shifts": [P, P, P, P, I64, P],
+    "fu_edge_shifts_batched": [P, P, P, P, I64, I32, P],
+    "fu_outer_sum3_batched": [P, P, P, P, P, I64, I64, I32, P],
     "fu_outer_sum3": [P, P, P, P, P, I64, I64, P],
     "fu_morton_keys": [P, P, P, I64, P],
     "fu_sort_pairs_i64": [P, P, P, P, I64, I32, I32, P, SZ_P, P],

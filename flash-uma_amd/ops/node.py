@@ -255,6 +255,51 @@ def edge_shifts(cell_offsets, cell):
     return EdgeShifts.apply(cell_offsets, cell)
 
 
+class EdgeShiftsBatched(torch.autograd.Function):
+    """shifts[e] = cell_offsets[e] @ cell[s] for the edges edge_ptr[s] .. edge_ptr[s + 1] of system s."""
+
+    @staticmethod
+    def forward(ctx, cell_offsets, cell, edge_ptr):
+        off = _lib.require(cell_offsets, torch.float32, "cell_offsets")
+        c = _lib.require(cell, torch.float32, "cell")
+        E, S = off.shape[0], c.shape[0]
+        shifts = torch.empty(E, 3, device=off.device, dtype=torch.float32)
+        _lib.call("fu_edge_shifts_batched", off.data_ptr(), c.data_ptr(), edge_ptr.data_ptr(), shifts.data_ptr(), E, S,
+                  _lib.stream_ptr(off.device))
+        ctx.save_for_backward(off, edge_ptr)
+        return shifts
+
+    @staticmethod
+    def backward(ctx, g_shifts):
+        off, edge_ptr = ctx.saved_tensors
+        g_shifts = g_shifts.contiguous()
+        S = edge_ptr.numel() - 1
+        g_cell = torch.empty(S, 3, 3, device=off.device, dtype=torch.float32)
+        partial = torch.empty(S * 144, device=off.device, dtype=torch.float64)
+        _lib.call("fu_outer_sum3_batched", off.data_ptr(), g_shifts.data_ptr(), edge_ptr.data_ptr(), g_cell.data_ptr(),
+                  partial.data_ptr(), partial.numel(), off.shape[0], S, _lib.stream_ptr(off.device))
+        return None, g_cell, None
+
+
+def edge_shifts_batched(cell_offsets, cell, nedges):
+    """shifts = cell_offsets @ cell of each edge's system: cell (S, 3, 3), nedges (S,) edges per system,
+    contiguous.  The kernel takes float32 cells and offsets without a gradient on the GPU; anything
+    else goes through torch.  The edge counts are read back once, as torch's repeat_interleave does."""
+    E = cell_offsets.shape[0]
+    if not (cell.is_cuda and cell.dtype == torch.float32 and cell.dim() == 3 and tuple(cell.shape[1:]) == (3, 3) and
+            tuple(cell_offsets.shape) == (E, 3) and cell_offsets.device == cell.device and
+            not cell_offsets.requires_grad and nedges.dtype == torch.int64 and nedges.device == cell.device and
+            nedges.shape == cell.shape[:1] and cell.shape[0] > 0):
+        cell_per_edge = cell.repeat_interleave(nedges, dim=0)
+        return torch.einsum("ij,ijk->ik", cell_offsets.to(cell_per_edge.dtype), cell_per_edge)
+    ptr = torch.zeros(nedges.numel() + 1, dtype=torch.int64, device=cell.device)
+    torch.cumsum(nedges, 0, out=ptr[1:])
+    total, least = torch.stack([ptr[-1], nedges.min()]).tolist()
+    if total != E or least < 0:
+        raise RuntimeError(f"edge_shifts_batched: nedges (sum {total}, least {least}) do not describe {E} edges")
+    return EdgeShiftsBatched.apply(cell_offsets, cell, ptr)
+
+
 def system_ptr(batch: torch.Tensor, n_systems: int) -> torch.Tensor:
     """(S + 1,) int32 segment pointers of a batch vector sorted ascending (atoms of system s
     are rows [ptr[s], ptr[s + 1]))."""

@@ -40,6 +40,8 @@ KERNEL_ENTRY = {
     "linear_rows16_kernel": "fu_linear_batched",
     "gate_fwd_kernel": "fu_gate_act_fwd", "gate_bwd_kernel": "fu_gate_act_bwd",
     "gather_rows_kernel": "fu_gather_rows", "scatter_rows_kernel": "fu_scatter_rows",
+    "edge_shifts_batched_kernel": "fu_edge_shifts_batched", "outer_sum3_batched_stage1": "fu_outer_sum3_batched",
+    "outer_sum3_batched_stage2": "fu_outer_sum3_batched",
     "edge_shifts_kernel": "fu_edge_shifts", "outer_sum3_stage1": "fu_outer_sum3", "outer_sum3_stage2": "fu_outer_sum3",
     "balance_sums_kernel": "fu_balance_channels", "balance_apply_kernel": "fu_balance_channels",
     "morton_keys_kernel": "fu_morton_keys", "invert_perm_kernel": "fu_invert_perm", "take_i64_kernel": "fu_take_i64",

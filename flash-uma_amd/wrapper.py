@@ -12,7 +12,7 @@ import torch.nn.functional as F
 
 from model import eSCN_Inference_Model
 from node_layers import adopt_atom_wise, adopt_rms_norm
-from ops.node import edge_shifts
+from ops.node import edge_shifts, edge_shifts_batched
 
 
 @torch.no_grad()
@@ -148,8 +148,7 @@ class ZeroAllocBackbone(nn.Module):
         if len(data.natoms) == 1:
             shifts = edge_shifts(data.cell_offsets, data.cell)
         else:
-            cell_per_edge = data.cell.repeat_interleave(data.nedges, dim=0)
-            shifts = torch.einsum("ij,ijk->ik", data.cell_offsets.to(cell_per_edge.dtype), cell_per_edge)
+            shifts = edge_shifts_batched(data.cell_offsets, data.cell, data.nedges)
 
         x_node = self.ce(pos=data.pos, Z=data.atomic_numbers, batch=data.batch, edge_index=data.edge_index,
                          shifts=shifts, csd_emb=csd_mixed_emb, charge=data.charge, spin=data.spin,

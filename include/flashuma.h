@@ -545,6 +545,14 @@ int fu_scatter_rows(const float* src, const int64_t* idx, float* dst, int64_t ro
 int fu_edge_shifts(const float* cell_offsets, const float* cell, const int64_t* perm,
                    float* shifts, int64_t E, void* stream);
 
+/* The same for S systems (wrapper.py:193-194): edges edge_ptr[s] .. edge_ptr[s + 1] - 1 (edge_ptr S + 1
+ * int64, ascending from 0) with cells[s] (S x 3 x 3), and the cells' gradient: out (S x 3 x 3) =
+ * sum of A[e]^T B[e] over each system's edges, in fp64 with a fixed order; partial: 144 S doubles. */
+int fu_edge_shifts_batched(const float* cell_offsets, const float* cells, const int64_t* edge_ptr, float* shifts,
+                           int64_t E, int32_t S, void* stream);
+int fu_outer_sum3_batched(const float* A, const float* B, const int64_t* edge_ptr, float* out, double* partial,
+                          int64_t partial_len, int64_t E, int32_t S, void* stream);
+
 /* out (3x3) = sum_e A[perm_a[e]]^T B[e] over E rows of 3 (perm_a NULL = identity), in fp64
  * with a fixed two-stage order (deterministic); the cell gradient of the shifts product.
  * partial is a workspace of at least 256 * 9 doubles. */

@@ -172,3 +172,29 @@ def test_linear_batched_few_rows(cuda, M, N, K, batch):
     # fp32 products in sums of K / 4 terms, or 22-bit operands past the rule
     assert e <= 1e-6 and e <= 2.0 * t + 1e-7, (e, t)
     assert torch.equal(Y[..., N:].cpu(), R[..., N:])
+
+
+@pytest.mark.parametrize("counts", [[3, 0, 257, 1], [1], [0, 0, 5000, 70, 0], [40] * 300])
+def test_edge_shifts_batched(cuda, counts):
+    """Shifts of several systems and their cells' gradients against float64, with systems of no edges;
+    counts that do not describe the edges are refused; a float64 cell still works."""
+    from ops.node import edge_shifts_batched
+    g = torch.Generator().manual_seed(len(counts))
+    n, E = torch.tensor(counts), sum(counts)
+    off = torch.randint(-3, 4, (E, 3), generator=g).float()
+    cell, cot = torch.randn(len(counts), 3, 3, generator=g) * 8, torch.randn(E, 3, generator=g)
+    cd = cell.double().requires_grad_()
+    ref = torch.einsum("ij,ijk->ik", off.double(), cd.repeat_interleave(n, dim=0))
+    (gref,) = torch.autograd.grad(ref, cd, cot.double())
+    cg = cell.to(cuda).requires_grad_()
+    out = edge_shifts_batched(off.to(cuda), cg, n.to(cuda))
+    (gc,) = torch.autograd.grad(out, cg, cot.to(cuda))
+    # three fp32 products and two sums each; the gradient's sums in fp64, rounded once
+    assert (out.cpu().double() - ref.detach()).abs().max() <= 3 * 2.0 ** -23 * 3 * cell.abs().max() * 3
+    assert (gc.cpu().double() - gref).abs().max() <= 2.0 ** -22 * gref.abs().max()
+    assert torch.equal(gc, torch.autograd.grad(edge_shifts_batched(off.to(cuda), cg, n.to(cuda)), cg, cot.to(cuda))[0])
+    for bad in (n + torch.eye(len(counts), dtype=torch.long)[0], torch.cat([n[:-1], n[-1:] - 1])):
+        with pytest.raises(RuntimeError):
+            edge_shifts_batched(off.to(cuda), cg, bad.to(cuda))
+    d = edge_shifts_batched(off.to(cuda), cell.double().to(cuda), n.to(cuda))
+    assert d.dtype == torch.float64 and torch.allclose(d.cpu(), ref.detach(), atol=1e-12)
