@@ -12,7 +12,8 @@
 //  * split fp16 (default, F16): each staged row is scaled by its power of two and split into
 //    two fp16 planes (split_f16.h); three v_mfma_f32_32x32x16_f16 per 32x32 block and chunk.
 //    The scales come from the first chunk (from a pre-pass over the rows when K <= 64 or when a
-//    row's first chunk is zero); a tile whose accumulators came out non-finite (an fp16 piece
+//    weight row's first chunk is zero); a tile with a nonzero row of A whose first chunk is zero, or
+//    whose accumulators came out non-finite (an fp16 piece
 //    overflowed) runs its K loop again at exact scales.  The accumulators are unscaled before
 //    the epilogue.
 //  * split bf16: each staged fp32 element is split into three bf16 planes
@@ -521,7 +522,7 @@ __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_k
       };
       // one call site of the pass-0/1 loop (pass 0, or pass 1 after an exact scan); pass 2 has
       // its own two loops
-      bool exact = short_k;
+      bool exact = short_k, zeroA = false, zeroA2 = false;
       for (int pass = 0; pass < 2; ++pass) {
         if (!exact) {
           load_chunk(0);
@@ -531,7 +532,15 @@ __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_k
           eA = f16_exp_chunk(mA);
           if constexpr (TALL) eA2 = f16_exp_chunk(mA2);
           if constexpr (!WF) eW = f16_exp_chunk(mW);
-          exact = tile_bits(mA == 0.0f || mA2 == 0.0f || mW == 0.0f) != 0;
+          // A row of A with a zero first chunk gives no scale: its tile is accepted if the whole row is
+          // zero, which needs the pieces tracked.  Edges beyond the cutoff have such gradient rows; with
+          // 16 % of them every tile was scanned for exact scales first: 100,000 rows, N 768, K 640 538
+          // -> 370 us, N 128, K 1,536 310 -> 192 (without a pre-split weight 602 -> 385, 366 -> 206).
+          zeroA = mA == 0.0f;
+          zeroA2 = mA2 == 0.0f;
+          const unsigned z = tile_bits((zeroA || zeroA2 ? F16_LOW_A : 0u) | (mW == 0.0f ? F16_OVERFLOW : 0u));
+          exact = (z & F16_OVERFLOW) != 0;
+          track = track || (z & F16_LOW_A) != 0;
         }
         if (exact) {
           const bool two = f16_needs_exact(tile_bits(exact_scales()));
@@ -553,7 +562,7 @@ __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_k
         kloop(std::integral_constant<int, 0>{});
         if (exact) break;
         // every wave has left the loop (barrier above): its buffers may be restaged
-        bool bad = false;
+        bool bad = (zeroA && pmaxA > 0.0f) || (zeroA2 && pmaxA2 > 0.0f);
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll

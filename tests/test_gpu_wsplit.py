@@ -222,3 +222,25 @@ def test_weight_fragments_by_rows(cuda, M, N, K):
     assert torch.equal(y[5::31], b.expand_as(y[5::31]))
     if M < 4096:
         assert torch.equal(y, plain)
+
+
+@pytest.mark.parametrize("M", [3000, 5000, 70000])
+@pytest.mark.parametrize("later", [0.0, 1.0, 2.0 ** -40, 2.0 ** 30])
+def test_zero_first_chunks(cuda, M, later):
+    """Rows of A whose first 16 elements are zero: wholly zero ones (the tile keeps its first pass), and
+    ones whose later elements would not fit the scale such a row has there; 128-row tiles with and
+    without W2 and tall ones.  The other rows of their tiles lose nothing."""
+    _lib, linear = _ops()
+    N, K = 128, 384
+    g = torch.Generator().manual_seed(M)
+    x, W = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5
+    x[3::50, :16] = 0.0
+    x[3::50, 16:] *= later
+    x, W = x.to(cuda), W.to(cuda)
+    ref = x.double() @ W.double().T
+    rn = ref.norm(dim=1).clamp_min(1e-300)
+    fp32 = ((_fp32_mfma(x, W).double() - ref).norm(dim=1) / rn).max().item()
+    for y in (linear.gemm(x, W), _with_w2(x, W)):
+        assert torch.isfinite(y).all() and ((y[3::50] == 0.0).all() or later)
+        worst = ((y.double() - ref).norm(dim=1) / rn).max().item()
+        assert worst <= 1.5 * fp32 + 1e-7, (worst, fp32)
