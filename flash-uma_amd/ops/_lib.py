@@ -23,7 +23,7 @@ F32 = ctypes.c_float
 SZ_P = ctypes.POINTER(ctypes.c_size_t)
 
 # fu_version() of the library these signatures describe (major*10000 + minor*100 + patch).
-ABI_VERSION = 600
+ABI_VERSION = 700
 
 # Argument types of every exported entry point, in header order.
 SIGNATURES: dict[str, list] = {

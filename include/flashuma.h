@@ -42,7 +42,7 @@ extern "C" {
 #define FU_ERR_NULL (-5)        /* a required pointer is NULL */
 #define FU_ERR_WORKSPACE (-6)   /* the workspace is too small */
 
-/* Library version (major*10000 + minor*100 + patch): 600 (0.6.0) for the signatures in this
+/* Library version (major*10000 + minor*100 + patch): 700 (0.7.0) for the signatures in this
  * header.  0.2.0 added the int32 `accumulate` argument (before the stream) of fu_gather_bwd,
  * fu_scatter_bwd, fu_init_scatter_bwd, their _lmax forms and fu_complex_linear_gate(_bwd), and
  * dropped one pointer/stride pair of fu_linear_gate_bwd; 0.3.0 changed the layout and size of
@@ -51,8 +51,9 @@ extern "C" {
  * fu_linear_weight_split and fu_linear_resident (nothing changed); 0.5.0 added the W2 argument
  * (before the stream) of fu_linear, fu_linear_gate, fu_linear_gate_bwd and
  * fu_linear_dgrad_ln_silu_bwd; 0.6.0 added fu_radial_gather_fwd, fu_radial_gather_perm and
- * their _lmax forms (nothing changed).  A caller built against
- * another version must not call into this library. */
+ * their _lmax forms (nothing changed); 0.7.0 added fu_so2_pair_fwd, fu_so2_pair_bwd, fu_linear_short,
+ * fu_nlist_limits, fu_edge_shifts_batched and fu_outer_sum3_batched (nothing changed).  A caller built
+ * against another version must not call into this library. */
 int fu_version(void);
 
 /* Message of the last error returned on the calling host thread ("" if none). */
