@@ -246,21 +246,23 @@ __global__ __launch_bounds__(1024) void nlist_scan_kernel(const int32_t* __restr
   if (b1 == N && t == 0) row_ptr[N] = before;
 }
 
-// limits[0], limits[1] (zeroed by the caller) = the largest |wrap| and the largest count
+// limits[0], limits[1] (zeroed by the caller) = the largest |wrap| and the largest count.  Unsigned: a
+// coordinate 2^31 cells or more below the origin has the wrap -2^31, whose magnitude no int holds.
 __global__ __launch_bounds__(256) void nlist_limits_kernel(const int32_t* __restrict__ wrap,
                                                            const int32_t* __restrict__ count, int64_t N,
                                                            int64_t* __restrict__ limits) {
-  int m[2] = {0, 0};
+  unsigned m[2] = {0u, 0u};
   for (int64_t a = (int64_t)blockIdx.x * 256 + threadIdx.x; a < 3 * N; a += (int64_t)gridDim.x * 256) {
-    const int v = wrap[a], u = v < 0 ? (int)(0u - (unsigned)v) : v;
+    const int32_t v = wrap[a];
+    const unsigned u = v < 0 ? 0u - (unsigned)v : (unsigned)v;
     m[0] = u > m[0] ? u : m[0];
-    if (a < N) m[1] = count[a] > m[1] ? count[a] : m[1];
+    if (a < N) m[1] = (unsigned)count[a] > m[1] ? (unsigned)count[a] : m[1];
   }
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
     for (int s = 1; s < 64; s <<= 1) {
-      const int v = __shfl_xor(m[h], s, 64);
+      const unsigned v = (unsigned)__shfl_xor((int)m[h], s, 64);
       m[h] = v > m[h] ? v : m[h];
     }
     if ((threadIdx.x & 63) == 0 && m[h] > 0)

@@ -196,3 +196,27 @@ def test_radius_graph_many_bins(cuda, n, a, pbc):
     ei, off = systems.neighbor_list(pos, cell, pbc, 6.0, 30)
     gi, go = radius_graph(torch.from_numpy(pos).to(cuda), cell, pbc, 6.0, 30)
     assert np.array_equal(gi.cpu().numpy(), ei) and np.array_equal(go.cpu().numpy(), off)
+
+
+@pytest.mark.parametrize("wrap", [-2 ** 31, 2 ** 31 - 1, -61, 60])
+def test_nlist_limits_of_saturated_wraps(cuda, wrap):
+    """A single wrap among zeros, at the ends of its type: its magnitude as a 64-bit number."""
+    from ops import _lib
+    N = 700
+    w = torch.zeros(N, 3, dtype=torch.int32, device=cuda)
+    w[431, 1] = wrap
+    count = torch.zeros(N, dtype=torch.int32, device=cuda)
+    lim = torch.zeros(2, dtype=torch.int64, device=cuda)
+    _lib.call("fu_nlist_limits", w.data_ptr(), count.data_ptr(), N, lim.data_ptr(), _lib.stream_ptr(cuda))
+    assert lim.tolist() == [abs(wrap), 0]
+
+
+@pytest.mark.parametrize("far", [-1e30, 1e30, float("-inf"), float("inf"), -700.0])
+def test_radius_graph_refuses_far_atoms(cuda, far):
+    """One atom too far outside the cell, below or above it, among ordinary ones: refused."""
+    from ops import _lib
+    from ops.neighbors import radius_graph
+    pos = torch.rand(40, 3, generator=torch.Generator().manual_seed(1)) * 11.0
+    pos[17, 2] = far
+    with pytest.raises(_lib.FlashUMAError, match="too far outside"):
+        radius_graph(pos.to(cuda), np.eye(3, dtype=np.float32) * 11.0, (True, True, True), 6.0, 30)
