@@ -276,7 +276,15 @@ __device__ __forceinline__ void complex_part(const Prob& p, int64_t row0, int n_
 #pragma unroll
         for (int r = 0; r < 16; ++r) T[op][r] *= rs[r];
     }
-    const bool two = lowW || (roughW && __any(f16_lossy(mr * f) || f16_lossy(mi * f)));
+    // pieces of 4 of a_r and of a_i, as in the tiled kernel: a run of 4 below the window next to
+    // normal elements counts
+    bool two = lowW;
+    if (roughW) {
+      bool low = false;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) low = low || f16_lossy(amax4(xr[h]) * f) || f16_lossy(amax4(xi[h]) * f);
+      two = two || __any(low);
+    }
     if (two) {   // pass 2 of split_f16.h, as in real_part
 #pragma unroll
       for (int op = 0; op < 3; ++op) {

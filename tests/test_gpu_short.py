@@ -8,9 +8,10 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _pair(cuda, M, C, L, ramp=0.0):
+def _pair(cuda, M, C, L, ramp=0.0, runs=0):
     """A pair on the GPU; with ramp > 0 the operands' columns carry 2^t and the weights' 2^-t, t
-    ramping over [-ramp, ramp] along K: the same products, opposite magnitudes."""
+    ramping over [-ramp, ramp] along K: the same products, opposite magnitudes.  runs > 0: t is -runs
+    on every other run of 4 columns of the m = 1, 2 operands, and 0 on the others."""
     from ops import gating
     from ops.linear import complex_weight_split, linear_weight_split
     g = torch.Generator().manual_seed(M + 7 * C + L)
@@ -23,6 +24,11 @@ def _pair(cuda, M, C, L, ramp=0.0):
     R1, I1, R2, I2 = w(n1, 2 * n1), w(n1, 2 * n1), w(n2, 2 * n2), w(n2, 2 * n2)
     S1, T1, S2, T2 = w(n1, n1), w(n1, n1), w(n2, n2), w(n2, n2)
     f0, f1, f2 = t(2 * n0), t(2 * n1), t(2 * n2)
+    if runs:
+        f1, f2 = (torch.exp2(-runs * (torch.arange(k) // 4 % 2).float()) for k in (2 * n1, 2 * n2))
+        # the last pieces of the weights small: rough columns, against which small operands count
+        for w_ in (R1, I1, R2, I2):
+            w_[:, -16:] *= 2.0 ** -10
     Xs = [X[0] * f0, X[1] * torch.cat([f1, f1]), X[2] * torch.cat([f2, f2])]
     rows = gating.gate_paired_rows(C, L)
     d = lambda a: a.contiguous().to(cuda)
@@ -77,6 +83,21 @@ def test_short_pair(cuda, monkeypatch, M, C, L, ramp):
     assert calls == ["fu_so2_pair_fwd", "fu_so2_pair_bwd"]
     again = _run(X, conv1, conv2, C, sp, cot)
     assert all(torch.equal(a, b) for a, b in zip(got, again))
+    monkeypatch.setattr(gating, "SHORT_PAIR_MAX_EDGES", 0)
+    tiled = _run(X, conv1, conv2, C, sp, cot)
+    for e, t in zip(_err(got, ref), _err(tiled, ref)):
+        assert e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
+
+
+@pytest.mark.parametrize("M,C,L", [(70, 128, 2), (33, 64, 3), (40, 64, 4)])
+@pytest.mark.parametrize("runs", [12, 20, 24])
+def test_short_pair_runs_of_four(cuda, monkeypatch, M, C, L, runs):
+    """Operands of the complex products with a run of 4 small elements in every piece of 8, against
+    weights as much larger there: those runs are below the fp16 window from 2^-16 on and go to the
+    two-loop products, as in the tiled kernels.  Bars of test_short_pair."""
+    from ops import gating
+    X, conv1, conv2, sp, cot, ref = _pair(cuda, M, C, L, runs=runs)
+    got = _run(X, conv1, conv2, C, sp, cot)
     monkeypatch.setattr(gating, "SHORT_PAIR_MAX_EDGES", 0)
     tiled = _run(X, conv1, conv2, C, sp, cot)
     for e, t in zip(_err(got, ref), _err(tiled, ref)):
