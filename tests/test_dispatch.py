@@ -1,0 +1,78 @@
+"""Which entry point a call goes to, and which calls are refused, by shapes and alignment: on the CPU,
+with the library's entry points replaced by a recorder (nothing is launched)."""
+import pytest
+import torch
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """Names of the entry points called; CPU tensors pass for device ones."""
+    from ops import _lib
+    names = []
+    monkeypatch.setattr(_lib, "call", lambda name, *a: names.append(name))
+    monkeypatch.setattr(_lib, "require", lambda t, dtype, name: t.to(dtype).contiguous())
+    monkeypatch.setattr(_lib, "ptr", lambda t: None if t is None else t.data_ptr())
+    monkeypatch.setattr(_lib, "stream_ptr", lambda device=None: 0)
+    monkeypatch.setattr(_lib, "side_stream", lambda device: None)
+    monkeypatch.setattr(_lib, "get_matmul_mode", lambda: _lib.MATMUL_SPLIT_F16)
+    return names
+
+
+def _pair(E=8, C=64, L=2, S=None, H=None, wide=0):
+    """Operands of a pair of E edges: S input channels per degree, H output ones (both C by default),
+    `wide` unused columns after X_m0's."""
+    S, H = S or C, H or C
+    n = (L + 1, L, L - 1)
+    z = torch.zeros
+    w = lambda r, k: (z(r, k), z(k, r))
+    cx = lambda r, k: (z(r, k), z(r, k), z(k, r), z(k, r))
+    W0, W0t = w((2 * L + 1) * C, 2 * n[0] * S)
+    V0, V0t = w(n[0] * H, n[0] * C)
+    conv1 = (W0, z((2 * L + 1) * C), W0t, *cx(n[1] * C, 2 * n[1] * S), *cx(n[2] * C, 2 * n[2] * S))
+    conv2 = (V0, z(n[0] * H), V0t, *cx(n[1] * H, n[1] * C), *cx(n[2] * H, n[2] * C))
+    X = [z(E, 2 * n[0] * S + wide), z(E, 4 * n[1] * S), z(E, 4 * n[2] * S)]
+    g = [z(E, n[0] * H), z(E, 2 * n[1] * H), z(E, 2 * n[2] * H)]
+    Y = (z(E, (2 * L + 1) * C), z(E, 2 * n[1] * C), z(E, 2 * n[2] * C))
+    return X, g, Y, conv1, conv2, tuple(z(4) for _ in range(12))
+
+
+SHORT, TILED = "fu_so2_pair_fwd", "fu_linear_gate"
+
+
+@pytest.mark.parametrize("C,L", [(64, 2), (128, 3), (192, 4), (256, 2)])
+def test_pair_takes_the_few_row_kernels(calls, C, L):
+    from ops import gating
+    X, g, Y, conv1, conv2, sp = _pair(C=C, L=L)
+    gating.conv_pair_fwd(X, conv1, conv2, C, sp)
+    gating.conv_pair_bwd(Y, conv1, conv2, C, sp, g)
+    assert calls == ["fu_so2_pair_fwd", "fu_so2_pair_bwd"]
+
+
+@pytest.mark.parametrize("form", [dict(S=32), dict(S=128), dict(H=32), dict(H=128), dict(wide=4)])
+def test_pair_of_other_widths_stays_tiled(calls, form):
+    """Input or output channels other than C, or rows with more columns than the weight reads: the few-row
+    entry points, which are given C alone, would read and write at other strides than the arrays'."""
+    from ops import gating
+    X, g, Y, conv1, conv2, sp = _pair(**form)
+    gating.conv_pair_fwd(X, conv1, conv2, 64, sp)
+    assert SHORT not in calls and TILED in calls
+    if "wide" not in form:
+        gating.conv_pair_bwd(Y, conv1, conv2, 64, sp, g)
+        assert "fu_so2_pair_bwd" not in calls and "fu_linear_gate_bwd" in calls
+
+
+def test_pair_with_an_unaligned_conv2_bias_stays_tiled(calls):
+    """fu_linear reads its bias a float at a time; the few-row kernels read 16 bytes."""
+    from ops import gating
+    X, g, Y, conv1, conv2, sp = _pair()
+    conv2 = (conv2[0], torch.zeros(conv2[1].numel() + 1)[1:], *conv2[2:])
+    gating.conv_pair_fwd(X, conv1, conv2, 64, sp)
+    assert SHORT not in calls and TILED in calls
+
+
+def test_pair_with_rows_of_another_count_stays_tiled(calls):
+    from ops import gating
+    X, g, Y, conv1, conv2, sp = _pair()
+    X[0] = X[0][:5]
+    gating.conv_pair_fwd(X, conv1, conv2, 64, sp)
+    assert SHORT not in calls
