@@ -196,27 +196,29 @@ SHORT_PAIR_MAX_FLOPS = 2.2e10
 SHORT_PAIR_MAX_EDGES = 16384
 
 
-@functools.lru_cache(maxsize=None)
+@functools.lru_cache(maxsize=64)
 def _pair_shapes(C: int, L: int):
-    """What the few-row entry points take a pair's arrays to be (they are given C, lmax and pointers): the
-    widths of X_m and g_Zo_m, and the shapes of the weights (W0, P1, P2, V0, R1, R2) and of their
-    transposes."""
+    """What the few-row entry points take a pair's arrays to be (they are given C, lmax and pointers): flops
+    of the forward products per edge (0: C or lmax not served), widths of X_m, shapes of W0, P1, P2, V0,
+    R1, R2; and the same with g_Zo_m and the transposed weights."""
     n = (L + 1, L, L - 1)
+    served = C % 64 == 0 and 0 < C <= 256 and 2 <= L <= 4
+    flops = served * C * C * (2 * ((2 * L + 1) * 2 * n[0] + n[0] * n[0]) + 18 * (L * L + n[2] * n[2]))
     fwd = [((2 * L + 1) * C, 2 * n[0] * C)] + [(n[m] * C, 2 * n[m] * C) for m in (1, 2)] + [(k * C, k * C) for k in n]
-    return ([2 * n[0] * C, 4 * n[1] * C, 4 * n[2] * C], [n[0] * C, 2 * n[1] * C, 2 * n[2] * C], fwd,
-            [(k, r) for r, k in fwd])
+    return ((flops, (2 * n[0] * C, 4 * n[1] * C, 4 * n[2] * C), tuple(fwd)),
+            (flops, (n[0] * C, 2 * n[1] * C, 2 * n[2] * C), tuple((k, r) for r, k in fwd)))
 
 
-def _short_pair(E: int, C: int, L: int, sp: tuple, arrays, widths, weights, shapes, *biases) -> bool:
-    """Whether the few-row kernels take a pair of E edges: split-fp16 mode, every weight pre-split, both
-    m = 0 biases present and 16-byte aligned, and arrays and weights of the pair's own shapes (another
-    number of input or output channels, wider arrays and an unaligned conv2 bias are the tiled kernels')."""
-    mac = 2 * ((2 * L + 1) * 2 * (L + 1) + (L + 1) ** 2) + 18 * (L * L + (L - 1) ** 2)   # flops / C^2
-    return (0 < E <= min(SHORT_PAIR_MAX_EDGES, SHORT_PAIR_MAX_FLOPS / (mac * C * C)) and C % 64 == 0 and C <= 256
-            and 2 <= L <= 4 and all(t is not None for t in sp + biases)
-            and all(b.data_ptr() % 16 == 0 for b in biases)
-            and all(x.shape == (E, w) for x, w in zip(arrays, widths))
-            and all(W.shape == s for W, s in zip(weights, shapes))
+def _short_pair(E: int, pair: tuple, sp: tuple, arrays, weights, *biases) -> bool:
+    """Whether the few-row kernels take a pair of E edges (pair: a half of _pair_shapes): split-fp16 mode,
+    every weight pre-split, both m = 0 biases present and 16-byte aligned, and arrays and weights of the
+    pair's own shapes (another number of input or output channels, wider arrays and an unaligned conv2
+    bias are the tiled kernels')."""
+    flops, (w0, w1, w2), shapes = pair
+    return (0 < E <= SHORT_PAIR_MAX_EDGES and 0 < E * flops <= SHORT_PAIR_MAX_FLOPS
+            and tuple([x.shape for x in arrays]) == ((E, w0), (E, w1), (E, w2))
+            and tuple([W.shape for W in weights]) == shapes and all([t is not None for t in sp])
+            and all([b is not None and b.data_ptr() % 16 == 0 for b in biases])
             and _lib.get_matmul_mode() == _lib.MATMUL_SPLIT_F16)
 
 
@@ -237,8 +239,7 @@ def conv_pair_fwd(X: list, conv1, conv2, C: int, splits, m0=None):
     dev = X[1].device
     L = _degrees(W0, C)
     sp = _splits12(splits)
-    xw, _, shapes, _ = _pair_shapes(C, L)
-    if m0 is None and _short_pair(X[1].shape[0], C, L, sp, X, xw, (W0, P1, P2, V0, R1, R2), shapes, b0, c0):
+    if m0 is None and _short_pair(X[1].shape[0], _pair_shapes(C, L)[0], sp, X, (W0, P1, P2, V0, R1, R2), b0, c0):
         X0, X1, X2 = (_lib.require(x, torch.float32, "X_m") for x in X)
         X[0] = X[1] = X[2] = None
         E = X1.shape[0]
@@ -298,8 +299,7 @@ def conv_pair_bwd(Y, conv1, conv2, C: int, splits, g: list):
     g1 = torch.zeros(E, 2 * L * C, device=dev) if g[1] is None else g[1].contiguous()
     g2 = torch.zeros(E, 2 * (L - 1) * C, device=dev) if g[2] is None else g[2].contiguous()
     g[0] = g[1] = g[2] = None
-    _, gw, _, shapes_t = _pair_shapes(C, L)
-    if _short_pair(E, C, L, sp, (g0, g1, g2), gw, (W0t, P1t, P2t, V0t, R1t, R2t), shapes_t):
+    if _short_pair(E, _pair_shapes(C, L)[1], sp, (g0, g1, g2), (W0t, P1t, P2t, V0t, R1t, R2t)):
         outs = [f(E, n * C) for n in (2 * L + 1, 2 * L, 2 * L - 2, L, L - 1, 2 * L + 2, 4 * L, 4 * L - 4)]
         _lib.call("fu_so2_pair_bwd", *(t.data_ptr() for t in (g0, g1, g2, Y0, Y1, Y2, sp[9], sp[1], sp[3], sp[11],
                                                               sp[5], sp[7], *outs)), E, C, L, st)
