@@ -88,6 +88,9 @@ def _scalar_gemm(x: torch.Tensor, W: torch.Tensor, b: torch.Tensor | None, add_t
     """x[:, 0] @ W^T (+ b) of x (N, K, Cin) or (N, Cin), or, with add_to (N, K, Cout), add_to[:, 0] += it in
     place (the residual of the GEMM's epilogue)."""
     N, O, I = x.shape[0], W.shape[0], W.shape[1]
+    if x.shape[-1] != I or (add_to is not None and (add_to.shape[0] != N or add_to.shape[-1] != O)):
+        raise _lib.FlashUMAError(f"scalar_gemm_so3: x {tuple(x.shape)} against W {tuple(W.shape)}" +
+                                 ("" if add_to is None else f", added to {tuple(add_to.shape)}"))
     y = torch.empty(N, O, device=x.device, dtype=torch.float32) if add_to is None else add_to
     _lib.call("fu_linear_batched", x.data_ptr(), x.stride(0), 0, W.data_ptr(), W.stride(0), 0, _lib.ptr(b), 0, 1,
               None if add_to is None else y.data_ptr(), y.stride(0), 0, y.data_ptr(), y.stride(0), 0, N, O, I, 1,

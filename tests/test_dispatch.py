@@ -76,3 +76,20 @@ def test_pair_with_rows_of_another_count_stays_tiled(calls):
     X[0] = X[0][:5]
     gating.conv_pair_fwd(X, conv1, conv2, 64, sp)
     assert SHORT not in calls
+
+
+def test_scalar_gemm_refuses_other_widths(calls):
+    """The scalar linear reads rows of x (N, K, Cin) at its own weight's width: a weight of another width is
+    refused, forward and backward, as ops.linear.gemm refuses it, not read across coefficients."""
+    from ops import _lib, node
+    z = torch.zeros
+    x, Wk, Wtk = z(5, 9, 64), z(9, 32, 64), z(9, 64, 32)
+    ok = node.scalar_gemm_so3(x, z(96, 64), z(96), z(64, 96), Wk, Wtk, z(32))
+    assert [t.shape for t in ok] == [(5, 96), (5, 9, 32)]
+    with pytest.raises(_lib.FlashUMAError):
+        node.scalar_gemm_so3(x, z(96, 128), z(96), z(128, 96), Wk, Wtk, z(32))
+    for Wt in (z(64, 64), z(128, 96)):   # of another gradient's width, and of another x's
+        xg = x.clone().requires_grad_()
+        pre, h = node.scalar_gemm_so3(xg, z(96, 64), z(96), Wt, Wk, Wtk, z(32))
+        with pytest.raises(_lib.FlashUMAError):
+            torch.autograd.grad((pre.sum() + h.sum()), xg)
