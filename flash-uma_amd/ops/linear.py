@@ -88,10 +88,10 @@ FEW_ROWS_MAX = 49152
 
 def gemm_few_rows(x: torch.Tensor, W: torch.Tensor, W2: torch.Tensor | None, out: torch.Tensor) -> torch.Tensor:
     """out = x W^T, on the few-row kernel (fu_linear_short, split-fp16 mode, W pre-split as W2, N =
-    64) up to FEW_ROWS_MAX rows, on fu_linear otherwise."""
+    64) up to FEW_ROWS_MAX rows of unit column stride, on fu_linear otherwise."""
     (M, K), N = x.shape, W.shape[0]
-    if (W2 is None or not 0 < M <= FEW_ROWS_MAX or N != 64 or x.stride(0) % 4 or x.data_ptr() % 16
-            or _lib.get_matmul_mode() != _lib.MATMUL_SPLIT_F16):
+    if (W2 is None or not 0 < M <= FEW_ROWS_MAX or N != 64 or W.shape[1] != K or x.stride(1) != 1 or x.stride(0) % 4
+            or x.data_ptr() % 16 or _lib.get_matmul_mode() != _lib.MATMUL_SPLIT_F16):
         return gemm(x, W, None, out, W2)
     _lib.call("fu_linear_short", x.data_ptr(), x.stride(0), W2.data_ptr(), None, out.data_ptr(), out.stride(0), M, N, K,
               _lib.stream_ptr(x.device))

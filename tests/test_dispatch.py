@@ -93,3 +93,19 @@ def test_scalar_gemm_refuses_other_widths(calls):
         pre, h = node.scalar_gemm_so3(xg, z(96, 64), z(96), Wt, Wk, Wtk, z(32))
         with pytest.raises(_lib.FlashUMAError):
             torch.autograd.grad((pre.sum() + h.sum()), xg)
+
+
+def test_few_row_product_dispatch(calls):
+    """fu_linear_short takes rows of unit column stride at the weight's width; other rows are copied for
+    fu_linear, and another width is refused."""
+    from ops import _lib, linear
+    z = torch.zeros
+    W, W2, out = z(64, 320), z(4), z(7, 64)
+    linear.gemm_few_rows(z(7, 320), W, W2, out)
+    linear.gemm_few_rows(z(7, 324)[:, :320], W, W2, out)
+    assert calls == ["fu_linear_short"] * 2
+    linear.gemm_few_rows(z(7, 640)[:, ::2], W, W2, out)
+    linear.gemm_few_rows(z(320, 8).t()[:7], W, W2, out)
+    assert calls[2:] == ["fu_linear"] * 2
+    with pytest.raises(_lib.FlashUMAError):
+        linear.gemm_few_rows(z(7, 256), W, W2, out)
