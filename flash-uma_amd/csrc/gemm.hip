@@ -84,11 +84,15 @@ struct GateBwd {
 };
 
 // Residual added by the plain epilogue (MODE 0): Y += R, R with row stride ldr, batch stride sR.
+// R may be Y itself (same strides): a thread reads each element just before it writes it.
 struct Resid {
   const float* R;
   int64_t ldr;
   int64_t sR;
 };
+// The output pointer: restrict where nothing else reads what it writes (not MODE 0: R may be Y).
+template <int MODE>
+using OutPtr = std::conditional_t<MODE == 0, float*, float* __restrict__>;
 
 // LayerNorm + SiLU epilogues over groups of LN_D = 128 columns (the radial-MLP hidden layers,
 // ops/ln_silu.py:29-123, in the grouped form of fu_ln_silu_grouped_*).  Each N-tile is one
@@ -154,7 +158,7 @@ template <int MODE, bool SPLIT, bool KTAIL = false, bool TALL = false, bool GATH
 __global__ __launch_bounds__(256, SPLIT ? (TALL ? 2 : 3) : 4) void linear_mfma_kernel(const float* __restrict__ A, int64_t lda, int64_t sA,
                                                           const float* __restrict__ W, int64_t ldw, int64_t sW,
                                                           const float* __restrict__ bias, int64_t sBias,
-                                                          int32_t bias_batches, float* __restrict__ Y, int64_t ldy,
+                                                          int32_t bias_batches, OutPtr<MODE> Y, int64_t ldy,
                                                           int64_t sY, int64_t M, int32_t N, int32_t K,
                                                           int32_t n_tiles, int64_t total_tiles, GateOut go,
                                                           GateBwd gb, Resid rs, LnEpi ln,

@@ -293,7 +293,8 @@ int fu_linear(const float* A, int64_t lda, const float* W, int64_t ldw, const fl
  * Used for the per-degree SO(3) linears of the atom-wise FFN (W_b = the weight of the
  * degree of coefficient b, bias on l = 0 only) and the radial bank's second layers.  R
  * (NULL, or row stride ldr >= N, batch stride stride_r, 16-byte aligned) is a residual added
- * in the epilogue: the skip x_mid + atom_wise(...) of model.py:157 without a separate add. */
+ * in the epilogue: the skip x_mid + atom_wise(...) of model.py:157 without a separate add.  R may be
+ * Y itself with the same strides (Y += the product); otherwise Y overlaps no other operand. */
 int fu_linear_batched(const float* A, int64_t lda, int64_t stride_a, const float* W, int64_t ldw,
                       int64_t stride_w, const float* bias, int64_t stride_bias, int32_t bias_batches,
                       const float* R, int64_t ldr, int64_t stride_r, float* Y, int64_t ldy,

@@ -195,6 +195,23 @@ def test_linear_batched_few_rows(cuda, M, N, K, batch):
     assert torch.equal(Y[..., N:].cpu(), R[..., N:])
 
 
+@pytest.mark.parametrize("M,N,K,mode", [(54, 128, 128, "split_f16"), (8200, 128, 64, "split_f16"), (8200, 200, 36, "split_f16"),
+                                        (8200, 128, 64, "split_bf16"), (8200, 128, 64, "fp32"), (66000, 128, 128, "split_f16")])
+def test_linear_batched_residual_in_place(cuda, M, N, K, mode):
+    """R = Y (16-row, 128-row and tall tiles, a K tail, the three modes): the bits of the same call with the
+    residual in an array of its own."""
+    from ops import _lib
+    g = torch.Generator(device=cuda).manual_seed(M + K)
+    r = lambda *s: torch.randn(*s, device=cuda, generator=g)
+    A, W, R = r(M, K), r(N, K), r(M, N)
+    Y, out = R.clone(), torch.empty_like(R)
+    with _lib.matmul_mode(_lib.MATMUL_MODES[mode]):
+        for res, y in ((R, out), (Y, Y)):
+            _lib.call("fu_linear_batched", A.data_ptr(), K, 0, W.data_ptr(), K, 0, None, 0, 0, res.data_ptr(), N, 0,
+                      y.data_ptr(), N, 0, M, N, K, 1, _lib.stream_ptr(cuda))
+    assert torch.equal(Y, out)
+
+
 @pytest.mark.parametrize("counts", [[3, 0, 257, 1], [1], [0, 0, 5000, 70, 0], [40] * 300])
 def test_edge_shifts_batched(cuda, counts):
     """Shifts of several systems and their cells' gradients against float64, with systems of no edges;
