@@ -28,8 +28,9 @@
 //  1. exact scales, from a pass over the rows: e = 14 - floor(log2 R), R the row's largest
 //     magnitude (R 2^e in [2^14, 2^15)), so pieces down to 2^-17 R stay in the window.  Pass 0
 //     is skipped for rows of up to F16_PREPASS_CHUNKS chunks and for a tile with a zero first
-//     chunk of W (nothing to scale from), and not accepted for one with a row of A whose first chunk
-//     is zero but not the rest;
+//     chunk of W or a row of A that begins with zeros and is nonzero where the tile looks further on
+//     (nothing to scale from), and not accepted for one with any row of A whose first chunk is zero
+//     but not the rest;
 //  2. for a tile that pass 1 cannot hold (a piece below 2^-17 of its row's maximum against a
 //     rough other operand): exact scales, and the K loop runs twice, first with the products
 //     hi_a lo'_b + lo'_a hi_b of the residuals scaled up, lo' = fp16((x 2^e - hi) 2^11),

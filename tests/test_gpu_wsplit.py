@@ -244,3 +244,29 @@ def test_zero_first_chunks(cuda, M, later):
         assert torch.isfinite(y).all() and ((y[3::50] == 0.0).all() or later)
         worst = ((y.double() - ref).norm(dim=1) / rn).max().item()
         assert worst <= 1.5 * fp32 + 1e-7, (worst, fp32)
+
+
+@pytest.mark.parametrize("M,K", [(3000, 384), (3000, 100), (5000, 384), (70000, 384), (70000, 100)])
+@pytest.mark.parametrize("start", [16, 150, -16, -1], ids=["first_chunk", "first_third", "last_chunk_only", "one_element"])
+@pytest.mark.parametrize("later", [1.0, 2.0 ** -40, 2.0 ** 30])
+def test_rows_that_begin_with_zeros(cuda, M, K, start, later):
+    """Rows of A whose nonzero part is met by the tile's look at two further chunks, and ones whose part lies
+    elsewhere and is met after the first pass: the same bars, every row."""
+    _lib, linear = _ops()
+    N = 128
+    g = torch.Generator().manual_seed(M + K)
+    x, W = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g) / K ** 0.5
+    rows = x[3::50]
+    start = min(start, 60) if K == 100 else start
+    if start == -1:
+        rows[:, :] = torch.where(torch.arange(K) == 33, rows, torch.zeros(()))
+    else:
+        rows[:, :start] = 0.0
+    rows *= later
+    x, W = x.to(cuda), W.to(cuda)
+    ref = x.double() @ W.double().T
+    rn = ref.norm(dim=1).clamp_min(1e-300)
+    fp32 = ((_fp32_mfma(x, W).double() - ref).norm(dim=1) / rn).max().item()
+    for y in (linear.gemm(x, W),) + ((_with_w2(x, W),) if K % 16 == 0 else ()):
+        worst = ((y.double() - ref).norm(dim=1) / rn).max().item()
+        assert torch.isfinite(y).all() and worst <= 1.5 * fp32 + 1e-7, (worst, fp32)
