@@ -35,7 +35,7 @@ KERNEL_ENTRY = {
     "resident_weight_scale_kernel": "fu_linear_weight_split", "resident_weight_summary_kernel": "fu_linear_weight_split",
     "resident_weight_split_kernel": "fu_linear_weight_split", "linear_resident_kernel": "fu_linear_resident",
     "radial_gather_kernel": "fu_radial_gather_fwd", "radial_gather_lmax_kernel": "fu_radial_gather_fwd_lmax",
-    "short_kernel": "fu_so2_pair_fwd/bwd, fu_linear_short", "short_ln_bwd_kernel": "fu_linear_dgrad_ln_silu_bwd",
+    "short_kernel": "fu_so2_pair_fwd or _bwd", "short_ln_bwd_kernel": "fu_linear_dgrad_ln_silu_bwd",
     "rms_norm_fwd_kernel": "fu_rms_norm_sh_fwd", "rms_norm_bwd_kernel": "fu_rms_norm_sh_bwd",
     "linear_rows16_kernel": "fu_linear_batched",
     "gate_fwd_kernel": "fu_gate_act_fwd", "gate_bwd_kernel": "fu_gate_act_bwd",
@@ -60,6 +60,10 @@ KERNEL_ENTRY = {
 # GATHER: fu_gather_linear_gate); complex_linear_kernel<MODE, PATH, KTAIL>
 LINEAR_MODE = {"0": "fu_linear", "1": "fu_linear_gate", "2": "fu_linear_gate_bwd", "3": "fu_linear_ln_silu",
                "4": "fu_linear_ln_silu_bwd", "5": "fu_linear_dgrad_ln_silu_bwd"}
+# short_kernel<MODE, KIND>; the last launch of the pair is the same instance both ways (conv2 forward, the
+# conv1 input gradients backward)
+SHORT_KERNEL = {("0", "0"): "fu_linear_short", ("1", "0"): "fu_so2_pair_fwd", ("1", "1"): "fu_so2_pair_fwd",
+                ("2", "0"): "fu_so2_pair_bwd", ("2", "1"): "fu_so2_pair_bwd"}
 COMPLEX_MODE = {"0": "fu_complex_linear", "1": "fu_complex_linear_gate", "2": "fu_complex_linear_gate_bwd"}
 
 
@@ -80,6 +84,8 @@ def kernel_entry(kernel_name: str, grid_y: int = 1) -> str | None:
         if ent == "fu_linear" and grid_y > 1:
             return "fu_linear_batched"
         return ent
+    if base == "short_kernel":
+        return SHORT_KERNEL.get(tuple(targs[:2]), KERNEL_ENTRY[base])
     if base == "complex_linear_kernel":
         return COMPLEX_MODE.get(targs[0] if targs else "0")
     return KERNEL_ENTRY.get(base)

@@ -33,15 +33,23 @@ F16_PRODUCTS = 3                # fp16 products per fp32 product in the split-fp
 MATMUL_SPLIT_BF16, MATMUL_FP32, MATMUL_SPLIT_F16 = 0, 1, 2
 
 
-def _products(name: str, matmul_mode: int) -> tuple[int, str]:
-    """Matrix-core products per fp32 product of entry `name` in `matmul_mode`, and their kind."""
-    if name == "fu_linear_resident":   # split-fp16 in every mode
-        return F16_PRODUCTS, "fp16 mfma, 3 products per fp32 product"
-    if matmul_mode == MATMUL_FP32:
-        return 1, "fp32 mfma"
+def _rows16(a) -> bool:
+    """Whether a call of fu_linear_batched runs on its 16-row fp32 tiles (use_rows16 in csrc/gemm.hip)."""
+    M, N, K, B = a[15], a[16], a[17], a[18]
+    return (N % 16 == 0 and K % 32 == 0 and (B == 1 or M <= 512) and M <= 16 * 512
+            and -(-M // 16) * B * -(-N // 128) <= 512)
+
+
+def _products(name: str, args, matmul_mode: int) -> tuple[int, str, float]:
+    """Matrix-core products per fp32 product of a call of entry `name` in `matmul_mode`, their kind and
+    their peak (TFLOP/s)."""
+    if name in ("fu_linear_resident", "fu_linear_short"):   # split-fp16 in every mode
+        return F16_PRODUCTS, "fp16 mfma, 3 products per fp32 product", BF16_MFMA_PEAK_TFLOPS
+    if matmul_mode == MATMUL_FP32 or (name == "fu_linear_batched" and _rows16(args)):
+        return 1, "fp32 mfma", FP32_MFMA_PEAK_TFLOPS
     if matmul_mode == MATMUL_SPLIT_F16 and name != "fu_gather_linear_gate":
-        return F16_PRODUCTS, "fp16 mfma, 3 products per fp32 product"
-    return SPLIT_PRODUCTS, "bf16 mfma, 6 products per fp32 product"
+        return F16_PRODUCTS, "fp16 mfma, 3 products per fp32 product", BF16_MFMA_PEAK_TFLOPS
+    return SPLIT_PRODUCTS, "bf16 mfma, 6 products per fp32 product", BF16_MFMA_PEAK_TFLOPS
 
 
 def _gating_fwd(a):
@@ -218,6 +226,47 @@ def _linear_resident(a):
     return 4 * (M * K + M * N + N * K), 2 * M * N * K
 
 
+def _linear_short(a):
+    M, N, K = a[6], a[7], a[8]
+    return 4 * (M * K + M * N + N * K), 2 * M * N * K
+
+
+def _pair_flops(E, C, L):
+    """Forward (or input-gradient) products of a convolution pair: m = 0 real, m = 1, 2 complex with
+    three real products."""
+    return E * C * C * (2 * ((2 * L + 1) * 2 * (L + 1) + (L + 1) ** 2) + 18 * (L * L + (L - 1) ** 2))
+
+
+def _pair_weights(C, L):
+    return C * C * ((2 * L + 1) * 2 * (L + 1) + (L + 1) ** 2 + 6 * (L * L + (L - 1) ** 2))
+
+
+def _pair_fwd(a):
+    # X_m (2 (L+1) + 4 L + 4 (L-1) = 10 L - 2 blocks of C) read, Y_m (6 L - 1) and O_m (5 L - 1) written;
+    # the gated Z_m stay between the launches and are not counted
+    E, C, L = a[20], a[21], a[22]
+    return 4 * (E * C * (21 * L - 4) + _pair_weights(C, L)), _pair_flops(E, C, L)
+
+
+def _pair_bwd(a):
+    # g_Zo_m (5 L - 1 blocks) and Y_m (6 L - 1) read, g_X_m (10 L - 2) written; g_Y_m and the gate sums
+    # stay between the launches
+    E, C, L = a[20], a[21], a[22]
+    return 4 * (E * C * (21 * L - 4) + _pair_weights(C, L)), _pair_flops(E, C, L)
+
+
+def _shifts_batched(a):
+    # offsets read, shifts written; a cell and an edge pointer per system
+    E, S = a[4], a[5]
+    return 24 * E + 44 * S + 8, 0
+
+
+def _outer_sum_batched(a):
+    # both edge arrays read; a cell gradient written and an edge pointer read per system
+    E, S = a[6], a[7]
+    return 24 * E + 44 * S + 8, 0
+
+
 def _linear_batched(a):
     M, N, K, B = a[15], a[16], a[17], a[18]
     r = M * N if a[9] else 0   # the residual, read once
@@ -310,6 +359,11 @@ WORK = {
     "fu_linear": _linear,
     "fu_linear_batched": _linear_batched,
     "fu_linear_resident": _linear_resident,
+    "fu_linear_short": _linear_short,
+    "fu_so2_pair_fwd": _pair_fwd,
+    "fu_so2_pair_bwd": _pair_bwd,
+    "fu_edge_shifts_batched": _shifts_batched,
+    "fu_outer_sum3_batched": _outer_sum_batched,
     "fu_radial_gather_fwd": _radial_gather,
     "fu_radial_gather_fwd_lmax": _radial_gather_l,
     "fu_linear_ln_silu": _linear_ln_silu,
@@ -335,7 +389,8 @@ WORK = {
 
 MFMA_BOUND = {"fu_linear", "fu_linear_batched", "fu_complex_linear", "fu_linear_gate", "fu_complex_linear_gate",
               "fu_linear_gate_bwd", "fu_complex_linear_gate_bwd", "fu_linear_ln_silu", "fu_linear_ln_silu_bwd",
-              "fu_linear_dgrad_ln_silu_bwd", "fu_gather_linear_gate", "fu_linear_resident"}
+              "fu_linear_dgrad_ln_silu_bwd", "fu_gather_linear_gate", "fu_linear_resident", "fu_linear_short",
+              "fu_so2_pair_fwd", "fu_so2_pair_bwd"}
 
 
 def summarize(durations, matmul_mode: int = MATMUL_SPLIT_F16) -> dict:
@@ -348,20 +403,23 @@ def summarize(durations, matmul_mode: int = MATMUL_SPLIT_F16) -> dict:
     which differs from `frac` where a launch's arithmetic intensity puts it under the HBM
     slope (the K = 128 shapes, whose operands and output are as large as their work);
     `hbm_bound_launches` counts those launches."""
-    mpeak = FP32_MFMA_PEAK_TFLOPS if matmul_mode == MATMUL_FP32 else BF16_MFMA_PEAK_TFLOPS
     agg: dict = {}
     for name, args, ms in durations:
         if name not in WORK:
             continue
         nbytes, flops = WORK[name](args)
-        a = agg.setdefault(name, {"calls": 0, "ms": 0.0, "bytes": 0, "flops": 0, "ideal_s": 0.0, "hbm_bound": 0})
+        a = agg.setdefault(name, {"calls": 0, "ms": 0.0, "bytes": 0, "flops": 0, "ideal_s": 0.0, "hbm_bound": 0,
+                                  "executed": 0, "mfma_s": 0.0, "ops": {}})
         a["calls"] += 1
         a["ms"] += ms
         a["bytes"] += nbytes
         a["flops"] += flops
         if name in MFMA_BOUND:
-            mul = _products(name, matmul_mode)[0]
-            t_mfma, t_hbm = mul * flops / (mpeak * 1e12), nbytes / (HBM_PEAK_GBS * 1e9)
+            mul, op, peak = _products(name, args, matmul_mode)
+            t_mfma, t_hbm = mul * flops / (peak * 1e12), nbytes / (HBM_PEAK_GBS * 1e9)
+            a["executed"] += mul * flops
+            a["mfma_s"] += t_mfma
+            a["ops"][op] = peak
             a["ideal_s"] += max(t_mfma, t_hbm)
             a["hbm_bound"] += int(t_hbm > t_mfma)
     out = {}
@@ -370,8 +428,10 @@ def summarize(durations, matmul_mode: int = MATMUL_SPLIT_F16) -> dict:
         rec = {"calls": a["calls"], "total_ms": round(a["ms"], 4), "avg_us": round(1e3 * a["ms"] / a["calls"], 2)}
         if name in MFMA_BOUND:
             fp32_rate = a["flops"] / sec / 1e12 if sec > 0 else 0.0
-            mul, op = _products(name, matmul_mode)
-            ach, peak = mul * fp32_rate, mpeak
+            ach = a["executed"] / sec / 1e12 if sec > 0 else 0.0
+            # one kind of product: its peak; several (16-row and 128-row tiles): the peak of their mix
+            op = " and ".join(sorted(a["ops"]))
+            peak = next(iter(a["ops"].values())) if len(a["ops"]) == 1 else round(a["executed"] / a["mfma_s"] / 1e12, 1)
             rec.update(bound="mfma", unit="TFLOP/s", achieved=round(ach, 2), peak=peak, frac=round(ach / peak, 4),
                        matrix_op=op, fp32_tflops=round(fp32_rate, 2), flops_per_launch=a["flops"] // a["calls"],
                        hbm_gbs=round(a["bytes"] / sec / 1e9, 1) if sec > 0 else 0.0,

@@ -85,3 +85,12 @@ def test_profiled_pass_table_from_a_trace(tmp_path):
     assert "| fu_complex_linear | 2.0 | 285.0 | 0.570 |" in text
     assert "kernels on 2 streams" in text
     assert "first dispatch to last completion 0.59 ms/step. The table" in text
+
+
+def test_few_row_instances_map_to_their_entry_points():
+    e = ps.kernel_entry
+    assert e("void fu::sg::short_kernel<0, 0>(fu::sg::Group)") == "fu_linear_short"
+    assert e("void fu::sg::short_kernel<1, 0>(x)") == e("void fu::sg::short_kernel<1, 1>(x)") == "fu_so2_pair_fwd"
+    assert e("void fu::sg::short_kernel<2, 0>(x)") == e("void fu::sg::short_kernel<2, 1>(x)") == "fu_so2_pair_bwd"
+    assert e("void fu::sg::short_kernel<0, 2>(x)") == "fu_so2_pair_fwd or _bwd"   # the same instance in both
+    assert e("void fu::sg::short_ln_bwd_kernel(x)") == "fu_linear_dgrad_ln_silu_bwd"

@@ -105,3 +105,66 @@ def test_accumulating_calls_count_the_read_back(name, sizes, per_edge):
     b0, _ = roofline.WORK[name](_args(name, **sizes, accumulate=0))
     b3, _ = roofline.WORK[name](_args(name, **sizes, accumulate=3))
     assert b3 - b0 == sizes["E"] * per_edge
+
+
+# entry points without a work function: set-up, graph building, queries, and node- or system-sized
+# copies and norms (none of them carries a step's edge work)
+UNCOUNTED = {
+    "fu_version", "fu_last_error", "fu_set_matmul_mode", "fu_matmul_mode", "fu_complex_weight_split_bytes",
+    "fu_complex_weight_split", "fu_linear_weight_split_bytes", "fu_linear_weight_split", "fu_radial_gather_perm",
+    "fu_radial_gather_perm_lmax", "fu_rms_norm_sh_fwd", "fu_rms_norm_sh_bwd", "fu_gate_act_fwd", "fu_gate_act_bwd",
+    "fu_balance_channels", "fu_balance_channels_noalloc", "fu_gather_rows", "fu_scatter_rows", "fu_edge_shifts",
+    "fu_outer_sum3", "fu_morton_keys", "fu_sort_pairs_i64", "fu_invert_perm", "fu_take_i64", "fu_csr_row_ptr",
+    "fu_narrow_i64_i32", "fu_nlist_bin", "fu_nlist_search", "fu_nlist_scan", "fu_nlist_limits", "fu_nlist_emit",
+    "fu_wigner_ext_width"}
+
+
+def test_every_entry_point_is_counted_or_named_as_not():
+    """A new entry point cannot drop out of the per-kernel table silently."""
+    import roofline
+    from ops import _lib
+    assert set(_lib.SIGNATURES) == set(roofline.WORK) | UNCOUNTED
+    assert not set(roofline.WORK) & UNCOUNTED
+
+
+@pytest.mark.parametrize("L,C,E", [(2, 128, 859), (3, 64, 77), (4, 256, 40)])
+def test_pair_work_is_that_of_its_tiled_calls(L, C, E):
+    """The pair's products are those of the tiled entry points it replaces, forward and backward; its bytes
+    leave out the gated Z (forward) and g_Y and the gate sums (backward), written and read in between."""
+    import roofline
+    W = lambda name, **s: roofline.WORK[name](_args(name, **s))
+    n = (L + 1, L, L - 1)
+    fwd = [W("fu_linear_gate", M=E, C=C, K=2 * n[0] * C, lmax=L), W("fu_linear", M=E, N=n[0] * C, K=n[0] * C)]
+    fwd += [W("fu_complex_linear_gate", M=E, Nc=k * C, Kc=2 * k * C) for k in n[1:]]
+    fwd += [W("fu_complex_linear", M=E, Nc=k * C, Kc=k * C) for k in n[1:]]
+    bwd = [W("fu_linear_gate_bwd", M=E, C=C, K=n[0] * C, lmax=L), W("fu_linear", M=E, N=2 * n[0] * C, K=(2 * L + 1) * C)]
+    bwd += [W("fu_complex_linear_gate_bwd", M=E, Nc=k * C, Kc=k * C) for k in n[1:]]
+    bwd += [W("fu_complex_linear", M=E, Nc=2 * k * C, Kc=k * C) for k in n[1:]]
+    for name, parts in (("fu_so2_pair_fwd", fwd), ("fu_so2_pair_bwd", bwd)):
+        nbytes, flops = W(name, E=E, C=C, lmax=L)
+        assert flops == sum(p[1] for p in parts)
+        assert 0 < nbytes < sum(p[0] for p in parts)
+        rec = roofline.summarize([(name, _args(name, E=E, C=C, lmax=L), 0.1)])[name]
+        assert rec["bound"] == "mfma" and "fp16" in rec["matrix_op"]
+
+
+def test_few_row_and_batched_shift_work():
+    import roofline
+    W = lambda name, **s: roofline.WORK[name](_args(name, **s))
+    assert W("fu_linear_short", M=900, N=64, K=640) == W("fu_linear", M=900, N=64, K=640)
+    assert W("fu_edge_shifts_batched", E=1000, S=7) == (24000 + 7 * 44 + 8, 0)
+    assert W("fu_outer_sum3_batched", E=1000, S=7) == (24000 + 7 * 44 + 8, 0)
+
+
+def test_sixteen_row_tiles_are_counted_as_fp32_products():
+    """fu_linear_batched on its 16-row tiles runs the fp32 matrix instructions; the line is the kernel's."""
+    import roofline
+    src = open(os.path.join(ROOT, "flash-uma_amd", "csrc", "gemm.hip")).read()
+    assert "ROWS16_MAX_GROUPS = 512, ROWS16_MAX_BATCHED_ROWS = 512;" in src
+    few, many = (_args("fu_linear_batched", M=m, N=128, K=128, batch=9) for m in (54, 8192))
+    r = roofline.summarize([("fu_linear_batched", few, 1.0)])["fu_linear_batched"]
+    assert r["matrix_op"] == "fp32 mfma" and r["peak"] == 157.3 and r["achieved"] == r["fp32_tflops"]
+    r = roofline.summarize([("fu_linear_batched", many, 1.0)])["fu_linear_batched"]
+    assert r["peak"] == 2500.0 and abs(r["achieved"] - 3 * r["fp32_tflops"]) < 0.01 + 1e-2 * r["achieved"]
+    r = roofline.summarize([("fu_linear_batched", few, 1.0), ("fu_linear_batched", many, 1.0)])["fu_linear_batched"]
+    assert 157.3 < r["peak"] < 2500.0 and "and" in r["matrix_op"]
