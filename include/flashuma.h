@@ -283,8 +283,9 @@ int fu_linear_dgrad_ln_silu_bwd(const float* A, int64_t lda, const float* W, int
  * the same weight pre-split by fu_linear_weight_split (16-byte aligned).  In matrix-core mode 2
  * with M >= 4,096 and K % 16 == 0 the kernel then loads its weight fragments from
  * W2 straight into registers (exact column scales and window flags from W2) instead of staging
- * and splitting W; otherwise W2 is not read.  No reference counterpart (an argument of this
- * build's kernels). */
+ * and splitting W; otherwise W2 is not read.  fu_linear_dgrad_ln_silu_bwd reads W2 instead of W at any
+ * M >= 1 in mode 2 with K % 16 == 0 (in the few-row kernel of fu_linear_short up to 24,576 rows).  No
+ * reference counterpart (an argument of this build's kernels). */
 int fu_linear(const float* A, int64_t lda, const float* W, int64_t ldw, const float* bias,
               float* Y, int64_t ldy, int64_t M, int32_t N, int32_t K, const void* W2, void* stream);
 

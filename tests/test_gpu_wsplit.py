@@ -1,14 +1,15 @@
-"""Tall split-fp16 GEMMs reading pre-split weight fragments (the W2 argument of fu_linear,
-fu_linear_gate, fu_linear_gate_bwd and fu_linear_dgrad_ln_silu_bwd): the products keep the bars
-of the tiled split GEMM against float64 and the fp32 MFMA (tests/test_gpu_ops.py), on the model's
-shapes and on the window cases of split_f16.h, and the model's users of W2 (the conv pair and the
-radial bank) agree with the same computation without it to fp32 rounding."""
+"""Split-fp16 GEMMs reading pre-split weight fragments (the W2 argument of fu_linear,
+fu_linear_gate, fu_linear_gate_bwd and fu_linear_dgrad_ln_silu_bwd), on 128-row and on tall tiles:
+the products keep the bars of the tiled split GEMM against float64 and the fp32 MFMA
+(tests/test_gpu_ops.py), on the model's shapes and on the window cases of split_f16.h, and the
+model's users of W2 (the conv pair and the radial bank) agree with the same computation without it
+to fp32 rounding."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
-M_TALL = 70000   # >= 65,536 rows: tall tiles, where W2 is read
+M_TALL = 70000   # >= 65,536 rows: tall tiles with and without W2
 
 
 def _ops():
@@ -104,33 +105,79 @@ def test_weight_fragments_dynamic_range(cuda):
     assert w_res <= 1.5 * w_f + 1e-7
 
 
-def test_w2_not_read_below_tall_tiles(cuda):
-    """Below 65,536 rows (128-row tiles) and outside the split-fp16 mode W2 is not read: the
-    result is the plain path's, bit for bit."""
+@pytest.mark.parametrize("M", [1, 3000, 4095])
+def test_w2_not_read_below_4096_rows(cuda, M):
+    """Below 4,096 rows fu_linear, fu_linear_gate and fu_linear_gate_bwd do not read W2, nor outside the
+    split-fp16 mode: with the fragments of another weight the result is the plain path's, bit for bit."""
     _lib, linear = _ops()
-    g = torch.Generator().manual_seed(9)
-    x = torch.randn(3000, 384, generator=g).to(cuda)
-    W = (torch.randn(256, 384, generator=g) / 384 ** 0.5).to(cuda)
-    W2 = linear.linear_weight_split(W)
-    assert torch.equal(linear.gemm(x, W, W2=W2), linear.gemm(x, W))
-    xt = torch.randn(M_TALL, 384, generator=g).to(cuda)
-    with _lib.matmul_mode(_lib.MATMUL_SPLIT_BF16):
-        assert torch.equal(linear.gemm(xt, W, W2=W2), linear.gemm(xt, W))
+    C, L = 64, 2
+    g = torch.Generator(device=cuda).manual_seed(M)
+    r = lambda *s: torch.randn(*s, device=cuda, generator=g)
+    x, W = r(M, 384), r(256, 384)
+    other = linear.linear_weight_split(r(256, 384))
+    assert torch.equal(linear.gemm(x, W, W2=other), linear.gemm(x, W))
+    if M == 3000:
+        xt = r(M_TALL, 384)
+        with _lib.matmul_mode(_lib.MATMUL_SPLIT_BF16):
+            assert torch.equal(linear.gemm(xt, W, W2=other), linear.gemm(xt, W))
+    n0, ny = (L + 1) * C, (2 * L + 1) * C
+    X0, W0, G, V0t, P1, P2 = r(M, 2 * n0), r(ny, 2 * n0), r(M, n0), r(n0, n0), r(M, L * C), r(M, (L - 1) * C)
+    st, res = _lib.stream_ptr(cuda), []
+    for w0, v0 in ((None, None), (linear.linear_weight_split(r(ny, 2 * n0)), linear.linear_weight_split(r(n0, n0)))):
+        Y0, Z0, gY0 = (torch.empty(M, n, device=cuda) for n in (ny, n0, ny))
+        _lib.call("fu_linear_gate", X0.data_ptr(), 2 * n0, W0.data_ptr(), 2 * n0, None, Y0.data_ptr(), ny, Z0.data_ptr(),
+                  n0, None, 0, M, C, 2 * n0, L, _lib.ptr(w0), st)
+        _lib.call("fu_linear_gate_bwd", G.data_ptr(), n0, V0t.data_ptr(), n0, Y0.data_ptr(), ny, P1.data_ptr(), L * C,
+                  P2.data_ptr(), (L - 1) * C, gY0.data_ptr(), ny, M, C, n0, L, _lib.ptr(v0), st)
+        res.append((Y0, Z0, gY0))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+
+
+@pytest.mark.parametrize("M,K", [(1, 1536), (24576, 384), (24577, 384), (30001, 1536), (65535, 384), (65536, 384)])
+def test_dgrad_ln_silu_reads_w2_at_any_rows(cuda, M, K):
+    """fu_linear_dgrad_ln_silu_bwd takes its product from W2 at every number of rows (the few-row kernel up
+    to 24,576, 128-row and tall tiles beyond): W itself may hold anything.  Against float64, and no worse
+    than 1.5x the tiles that read W."""
+    _lib, linear = _ops()
+    G, C, group = 3, 128, 1
+    g = torch.Generator(device=cuda).manual_seed(M + K)
+    r = lambda *s: torch.randn(*s, device=cuda, generator=g)
+    A, W, x = r(M, K), r(C, K) / K ** 0.5, r(M, G * C)
+    gm, bt = r(G * C).abs() + 0.5, r(G * C) * 0.1
+    xd = x.double().view(M, G, C)
+    mu = xd.mean(2).float().contiguous()
+    rs = (xd.var(2, unbiased=False) + 1e-5).rsqrt().float().contiguous()
+    s = slice(group * C, (group + 1) * C)
+    outs = []
+    for w, w2 in ((torch.full_like(W, float("nan")), linear.linear_weight_split(W)), (W, None)):
+        out = torch.empty(M, C, device=cuda)
+        _lib.call("fu_linear_dgrad_ln_silu_bwd", A.data_ptr(), K, w.data_ptr(), K, out.data_ptr(), C, M, K, x.data_ptr(),
+                  G * C, gm.data_ptr(), bt.data_ptr(), mu.data_ptr(), rs.data_ptr(), G, group, _lib.ptr(w2),
+                  _lib.stream_ptr(cuda))
+        outs.append(out)
+    v = x[:, s].double().requires_grad_()
+    xh = (v - v.mean(1, keepdim=True)) * (v.var(1, unbiased=False, keepdim=True) + 1e-5).rsqrt()
+    y = torch.nn.functional.silu(xh * gm[s].double() + bt[s].double())
+    (ref,) = torch.autograd.grad(y, v, A.double() @ W.double().T)
+    e, t = (_normwise(o, ref) for o in outs)
+    assert e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
 
 
 def _normwise(a, b):
     return ((a.double() - b.double()).norm() / b.double().norm()).item()
 
 
-def test_conv_pair_with_weight_fragments(cuda):
-    """conv1 + gate + conv2 and its backward at a tall size (C = 128, lmax 2) with the m = 0
-    weights pre-split (fu_linear_gate, fu_linear, fu_linear_gate_bwd read W2) against the same
+@pytest.mark.parametrize("M", [4095, 4096, 5001, 36863, 36865, 50001, M_TALL])
+def test_conv_pair_with_weight_fragments(cuda, monkeypatch, M):
+    """conv1 + gate + conv2 and its backward on the tiled kernels (C = 128, lmax 2), on both sides of the
+    lines of W2 and of its tall tiles and at a tall size, with the m = 0 weights pre-split (fu_linear_gate, fu_linear, fu_linear_gate_bwd read W2) against the same
     with the complex splits only: outputs and input gradients agree normwise to 2e-6, and the
     forward's first 2,048 rows match float64 at the op bar."""
     from ops import gating
     from ops.linear import complex_weight_split, linear_weight_split
     from oracle import ops_ref as R
-    C, L, M = 128, 2, M_TALL
+    monkeypatch.setattr(gating, "SHORT_PAIR_MAX_EDGES", 0)
+    C, L = 128, 2
     g = torch.Generator().manual_seed(11)
     r = lambda *s: torch.randn(*s, generator=g)
     X = [r(M, 2 * (L + 1) * C), r(M, 4 * L * C), r(M, 4 * (L - 1) * C)]
