@@ -46,8 +46,9 @@ def _assert_equal(ref, got):
 
 
 @pytest.mark.parametrize("layout", [0, 1])
-@pytest.mark.parametrize("E,N", [(70000, 2400), (3001, 200), (128, 7), (1, 1)])
+@pytest.mark.parametrize("E,N", [(70000, 2400), (49025, 1700), (49024, 1700), (3001, 200), (128, 7), (1, 1)])
 def test_radial_gather_bitwise(cuda, layout, E, N):
+    """49,024 edges are the last whose panels are shared by two workgroups, 49,025 the first that are not."""
     ops = _inputs(cuda, E, N, seed=E + N + layout)
     _assert_equal(*_both(*ops, layout))
 
@@ -130,9 +131,9 @@ def _lmax_inputs(cuda, E, N, L, seed):
 
 
 @pytest.mark.parametrize("L", [3, 4])
-@pytest.mark.parametrize("E,N", [(20000, 700), (1001, 64), (1, 1)])
+@pytest.mark.parametrize("E,N", [(50000, 1700), (49025, 1700), (49024, 1700), (20000, 700), (1001, 64), (1, 1)])
 def test_radial_gather_lmax_bitwise(cuda, L, E, N):
-    """fu_radial_gather_fwd_lmax against fu_linear_resident (unpermuted weight) followed by
+    """fu_radial_gather_fwd_lmax (panels of one workgroup from 49,025 edges on, shared below) against fu_linear_resident (unpermuted weight) followed by
     fu_gather_fwd_lmax (edge-parallel and node-centric forms): rad and X bitwise equal."""
     from ops import linear, lmax
     h2, W3, b3, x, idx_i, idx_j, wig, ext, csd, batch = _lmax_inputs(cuda, E, N, L, seed=7 * E + N + L)

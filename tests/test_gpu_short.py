@@ -138,6 +138,21 @@ def test_linear_short(cuda, M, N, K, ramp):
     assert (buf[:, N:] == 7.0).all() and e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
 
 
+@pytest.mark.parametrize("M,K", [(49152, 320), (49153, 320)])
+def test_few_row_product_on_both_sides_of_its_line(cuda, monkeypatch, M, K):
+    """gemm_few_rows at its last row count and past it: the two entry points, each at the bar above."""
+    from ops import _lib, linear
+    g = torch.Generator(device=cuda).manual_seed(M)
+    x, W = torch.randn(M, K, device=cuda, generator=g), torch.randn(64, K, device=cuda, generator=g) / K ** 0.5
+    calls, real = [], _lib.call
+    W2 = linear.linear_weight_split(W)
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    y = linear.gemm_few_rows(x, W, W2, torch.empty(M, 64, device=cuda))
+    assert calls == ["fu_linear_short" if M <= linear.FEW_ROWS_MAX else "fu_linear"]
+    ref = x.double() @ W.double().T
+    assert ((y.double() - ref).norm() / ref.norm()).item() <= 1e-6
+
+
 @pytest.mark.parametrize("M,K,group", [(1, 1536, 0), (31, 384, 4), (33, 1536, 2), (500, 3072, 1), (70, 16, 3)])
 def test_dgrad_ln_silu_short(cuda, M, K, group):
     """The radial output layer's input gradient with the LayerNorm-SiLU backward of its group, few rows
