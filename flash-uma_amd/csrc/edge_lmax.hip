@@ -21,7 +21,8 @@
 // wave64 per edge, lanes across channels, a contiguous XCD-aware edge range per workgroup; forward
 // scatters one wave per receiver with fp64 accumulators, segments in CSR order; backward gather
 // node-centric (one wave per CSR segment of the node, as receiver and as sender), so no kernel uses
-// atomics.  With few nodes two or four waves share a segment (node_waves, segment_waves).  The l blocks
+// atomics.  With few nodes two or four waves share a segment of the forward rotate-scatter and of the
+// gather backward (node_waves, segment_waves); the init scatter keeps one wave a node.  The l blocks
 // are processed one at a time to bound registers.
 #include "edge_lmax_layout.h"
 #include "fu_vec.h"

@@ -232,7 +232,7 @@ inline void with_waves(int w, F f) {
 }
 
 // Waves per segment of the gather backward, whose block already holds a wave per side; the rows of four
-// a side hold 154 KB of LDS at lmax 4, so only one block fits a CU.  As above:
+// a side hold 102 KB of LDS at lmax 4 and C = 128, so only one block fits a CU.  As above:
 //   nodes                      54            150           500           1000          1500
 //   lmax 2                   47|28|25      49| 31|29     77| 72| 73    145|136|136   206|201|198
 //   lmax 4                 163|92|73     172|101|80    225|161|179    297|296|338   499|431|487

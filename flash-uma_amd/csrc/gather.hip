@@ -351,7 +351,7 @@ __device__ __forceinline__ void gather_bwd_side(const float* __restrict__ gX0, c
 // C = 256 two edges in flight need more than the 170 registers of 3 waves per SIMD (449
 // spilled to scratch) or the 256 of 2 (116): one wave per SIMD keeps them in registers and
 // accumulation registers (2.26x faster at 245,760 edges: 5,160 -> 2,285 us).
-// W waves per segment (node_waves below): with few nodes each takes a contiguous part of the
+// W waves per segment (segment_waves in fu_vec.h): with few nodes each takes a contiguous part of the
 // segment, and the node gradients are added in part order, receiver parts first.
 template <int CPL, int L, int W>
 __global__ __launch_bounds__(128 * W, CPL >= 4 ? 1 : 3) void gather_bwd_kernel(

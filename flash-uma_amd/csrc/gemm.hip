@@ -1000,10 +1000,14 @@ void launch_short_ln_bwd(const float* A, int64_t lda, const void* W2, float* g_x
 using namespace fu;
 
 // Up to these many rows the radial output layers' input gradients (with a pre-split weight) run in
-// the few-row kernel of gemm_short.hip: its 32-row workgroups read the whole weight each, which
-// past that costs more than the 128-row tiles' idle CUs.  Measured, us, tiled / few-row: K = 1,536
-// 61 / 19 at 870 rows, 79 / 59 at 18,000, 82 / 85 at 30,000; K = 384 26 / 9, 31 / 28, 33 / 37;
-// K = 3,072 109 / 32, 145 / 104, 185 / 175.
+// the few-row kernel of gemm_short.hip: its 32-row workgroups, one a CU, read the whole weight each,
+// so its time steps up every 8,192 rows, and past three such rounds the 128-row tiles are faster.
+// us, few-row / tiles reading W2, captured:
+//   K       3,000 rows    9,000       18,000      24,576      27,000      30,000
+//   384       9 /  25    17 /  25    27 /  27    28 /  27    34 /  27    35 /  28
+//   1,536    20 /  59    38 /  62    55 /  63    57 /  63    73 /  64    74 /  64
+//   2,304    26 / 101    50 /  86    75 /  87    89 /  96   118 / 102   129 / 108
+//   3,072    33 / 132    64 / 111    98 / 113   130 / 144   168 / 144   170 / 159
 constexpr int64_t SHORT_LN_BWD_MAX_ROWS = 24576;
 
 // Rows from which the split mode uses tall (256-row) tiles: below it the 128-row tiles keep

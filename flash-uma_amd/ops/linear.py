@@ -79,10 +79,11 @@ def gemm_resident(x: torch.Tensor, W2: torch.Tensor, N: int, bias: torch.Tensor 
     return out
 
 
-# Up to this many rows a plain product of at most 64 columns with a pre-split weight runs in the
-# few-row kernel; the tiled kernels compute 128 columns there.  Measured, us, tiled / few-row, K = 640,
-# N = 64 (the Gaussian gradient of the radial trunk): 27 / 8.5 at 870 rows, 32 / 19 at 18,000, 33 /
-# 24 at 30,000, 44 / 40 at 60,000; K = 320 27 / 28 and K = 1,152 80 / 87 at 60,000.
+# Up to this many rows a plain product of 64 columns with a pre-split weight runs in the few-row kernel;
+# the tiled kernels compute 128 columns there.  Measured (the Gaussian gradient of the radial trunk), us,
+# few-row / tiles reading W2 at 6,000 | 30,000 | 49,152 | 60,000 rows: K = 192 5/11 | 12/12 | 16/21 | 20/21,
+# K = 320 6/14 | 15/18 | 21/27 | 26/28, K = 640 7/22 | 23/28 | 31/41 | 38/45, K = 1,152 12/40 | 35/44 |
+# 50/65 | 83/79.
 FEW_ROWS_MAX = 49152
 
 
