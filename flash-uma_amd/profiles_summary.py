@@ -5,6 +5,8 @@ command named in its header (run from the repository root on one MI355X):
 
   timed   per-kernel time over the timed steps of a bench.py kernel trace
           (--trace <dir>/<name>_kernel_trace.csv --warmup W --steps S)
+  cycles  per-kernel time over the passes of a program that repeats one call (--trace, --marker
+          a kernel of the call, --per-step its dispatches a pass)
   pmc     HBM bytes per launch from two counter passes, FETCH_SIZE and WRITE_SIZE, each run
           with --kernel-trace, scaled by what the counters read for the plain 256 MiB copy
           that bench.py --pmc-calibration dispatches first; also writes profiles/pmc_traffic.json
@@ -125,12 +127,7 @@ def timed(trace: str, warmup: int, steps: int, title: str, command: str, out: st
     sel = rows[starts[warmup + steps]:] if n_pass == 2 else timed_rows
     w0, w1 = int(timed_rows[0]["Start_Timestamp"]), max(int(r["End_Timestamp"]) for r in timed_rows)
     t0, t1 = int(sel[0]["Start_Timestamp"]), max(int(r["End_Timestamp"]) for r in sel)
-    agg = collections.defaultdict(lambda: [0, 0])
-    for r in sel:
-        key = (short_name(r["Kernel_Name"])[:90], kernel_entry(r["Kernel_Name"], _grid_y(r)))
-        agg[key][0] += 1
-        agg[key][1] += int(r["End_Timestamp"]) - int(r["Start_Timestamp"])
-    tot = sum(v[1] for v in agg.values())
+    agg, tot = _by_kernel(sel)
     lines = [f"# Kernel time per step — {title}", "", "Command (run from the repository root on one MI355X):", "",
              "```", command, "```", ""]
     if n_pass == 1:
@@ -150,7 +147,22 @@ def timed(trace: str, warmup: int, steps: int, title: str, command: str, out: st
                   f"{tot / 1e6 / steps:.2f} ms/step, first dispatch to last completion "
                   f"{(t1 - t0) / 1e6 / steps:.2f} ms/step. Summarised by "
                   f"`python flash-uma_amd/profiles_summary.py timed --pass profiled`.", ""]
-    lines += ["| ms/step | calls/step | avg us | share | kernel | entry point |", "|---:|---:|---:|---:|---|---|"]
+    _write(out, lines + _table(agg, tot, steps, top))
+
+
+def _by_kernel(sel: list[dict]) -> tuple[dict, int]:
+    """{(kernel, entry point): [launches, ns]} of trace rows and their total ns."""
+    agg = collections.defaultdict(lambda: [0, 0])
+    for r in sel:
+        key = (short_name(r["Kernel_Name"])[:90], kernel_entry(r["Kernel_Name"], _grid_y(r)))
+        agg[key][0] += 1
+        agg[key][1] += int(r["End_Timestamp"]) - int(r["Start_Timestamp"])
+    return agg, sum(v[1] for v in agg.values())
+
+
+def _table(agg: dict, tot: int, steps: int, top: int) -> list[str]:
+    """The table per kernel and the one per entry point."""
+    lines = ["| ms/step | calls/step | avg us | share | kernel | entry point |", "|---:|---:|---:|---:|---|---|"]
     for (nm, ent), (n, t) in sorted(agg.items(), key=lambda kv: -kv[1][1])[:top]:
         lines.append(f"| {t / 1e6 / steps:.3f} | {n / steps:.1f} | {t / n / 1e3:.1f} | {100 * t / tot:.1f}% | `{nm}` | "
                      f"{ent or '(torch / rocBLAS)'} |")
@@ -163,7 +175,27 @@ def timed(trace: str, warmup: int, steps: int, title: str, command: str, out: st
               "| entry point | calls/step | avg us | ms/step |", "|---|---:|---:|---:|"]
     for ent, (n, t) in sorted(by_entry.items(), key=lambda kv: -kv[1][1]):
         lines.append(f"| {ent} | {n / steps:.1f} | {t / n / 1e3:.1f} | {t / 1e6 / steps:.3f} |")
-    _write(out, lines)
+    return lines
+
+
+def cycles(trace: str, steps: int, marker: str, per_step: int, title: str, command: str, out: str,
+           top: int = 40) -> None:
+    """Kernel time per pass of a program that repeats one call: the last `steps` cycles from a marker
+    kernel (dispatched per_step times a pass) to the same one of the next pass, the last pass left out."""
+    rows = sorted(_read(trace), key=lambda r: int(r["Start_Timestamp"]))
+    starts = [i for i in _steps(rows, marker)][::-1]
+    if len(starts) < (steps + 1) * per_step:
+        raise SystemExit(f"{trace}: {len(starts)} dispatches of {marker}, {(steps + 1) * per_step} needed")
+    i0, i1 = starts[(steps + 1) * per_step - 1], starts[per_step - 1]
+    sel = rows[i0:i1]
+    wall = int(rows[i1]["Start_Timestamp"]) - int(rows[i0]["Start_Timestamp"])
+    agg, tot = _by_kernel(sel)
+    lines = [f"# Kernel time per pass — {title}", "", "Command (run from the repository root on one MI355X):", "", "```",
+             command, "```", "",
+             f"rocprofv3 kernel trace, {steps} passes, each from a `{marker}` dispatch to the one of the next pass: "
+             f"{len(sel) / steps:.0f} launches and {tot / 1e3 / steps:.0f} us of kernel time a pass; {wall / 1e3 / steps:.0f} us "
+             f"from pass to pass under the trace. Summarised by `python flash-uma_amd/profiles_summary.py cycles`.", ""]
+    _write(out, lines + _table(agg, tot, steps, top))
 
 
 def _joined(counters: str, trace: str) -> list[tuple[dict, int]]:
@@ -305,6 +337,11 @@ def main(argv=None) -> None:
     t.add_argument("--command", required=True)
     t.add_argument("--out", required=True)
     t.add_argument("--pass", dest="which", choices=("timed", "profiled"), default="timed")
+    c = sub.add_parser("cycles")
+    c.add_argument("--steps", type=int, required=True)
+    c.add_argument("--per-step", type=int, default=1)
+    for k in ("trace", "marker", "title", "command", "out"):
+        c.add_argument(f"--{k}", required=True)
     p = sub.add_parser("pmc")
     for k in ("fetch", "fetch-trace", "write", "write-trace", "config", "cmd-fetch", "cmd-write", "out", "commit"):
         p.add_argument(f"--{k}", required=True)
@@ -316,6 +353,8 @@ def main(argv=None) -> None:
     a = ap.parse_args(argv)
     if a.cmd == "timed":
         timed(a.trace, a.warmup, a.steps, a.title, a.command, a.out, which=a.which)
+    elif a.cmd == "cycles":
+        cycles(a.trace, a.steps, a.marker, a.per_step, a.title, a.command, a.out)
     elif a.cmd == "pmc":
         pmc(a.fetch, a.fetch_trace, a.write, a.write_trace, a.config, a.cmd_fetch, a.cmd_write, a.out, a.json,
             a.commit)

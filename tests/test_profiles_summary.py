@@ -94,3 +94,19 @@ def test_few_row_instances_map_to_their_entry_points():
     assert e("void fu::sg::short_kernel<2, 0>(x)") == e("void fu::sg::short_kernel<2, 1>(x)") == "fu_so2_pair_bwd"
     assert e("void fu::sg::short_kernel<0, 2>(x)") == "fu_so2_pair_fwd or _bwd"   # the same instance in both
     assert e("void fu::sg::short_ln_bwd_kernel(x)") == "fu_linear_dgrad_ln_silu_bwd"
+
+
+def test_cycles_table_from_a_trace(tmp_path):
+    """Three passes of a call that dispatches its marker twice: the two cycles before the last pass, each
+    with the kernels before and after the markers once."""
+    rows, t = [], 0
+    for name in ["void other(x)"] * 3 + ["void fu::edge_shifts_kernel(x)", "void fu::rms_norm_fwd_kernel<2>(x)",
+                                        "void fu::linear_rows16_kernel(x)", "void fu::rms_norm_fwd_kernel<2>(x)"] * 3:
+        rows.append((len(rows), name, t, t + 10000, 1))
+        t += 12000
+    tr, out = tmp_path / "t.csv", tmp_path / "t.md"
+    _trace(tr, rows)
+    ps.cycles(str(tr), 2, "rms_norm_fwd_kernel", 2, "test", "cmd", str(out))
+    text = out.read_text()
+    assert "4 launches and 40 us of kernel time a pass; 48 us from pass to pass" in text
+    assert "| fu_rms_norm_sh_fwd | 2.0 | 10.0 | 0.020 |" in text and "| fu_edge_shifts | 1.0 | 10.0 | 0.010 |" in text
