@@ -982,7 +982,8 @@ void launch_linear_rows16(const float* A, int64_t lda, int64_t sA, const float* 
 // fp32 rate cost more than the 128-row tiles' idle CUs.  Measured, us, 128 / 16 rows: nine products of
 // 128 x 128 10.9 / 6.2 at 54 rows (36 workgroups), 11.4 / 8.4 at 500 (288), 11.5 / 11.0 at 999 (567), 11.7 /
 // 16.8 at 2,000; 25 of them 11.5 / 8.7 at 250 (400), 11.6 / 14.2 at 500 (800); nine of 256 x 256 15.4 / 14.2
-// at 250 (288), 15.6 / 19.1 at 500 (576); one of 256 x 128 12.2 / 6.2 at 54, 13.1 / 8.7 at 4,000 (500).
+// at 250 (288), 15.6 / 19.1 at 500 (576); one of 256 x 128 12.2 / 6.2 at 54, 13.1 / 8.7 at 4,000 (500).  Even
+// at 512 workgroups for long or many products: K 512 23.7 / 23.0, K 1,024 40.2 / 41.4, 25 of 256 x 256 14.9 / 15.9.
 // Batches past 512 rows are the radial MLP's hidden layers, whose products fu_linear_ln_silu writes
 // too, from 128-row tiles: the two stay the same bit for bit.
 constexpr int64_t ROWS16_MAX_GROUPS = 512, ROWS16_MAX_BATCHED_ROWS = 512;
