@@ -71,7 +71,7 @@ constexpr bool pre_split(int path) { return path == CPATH_SPLIT3_PRE || path == 
 //    scale per output column n, shared by P, Q and S so that the three products stay
 //    combinable), then the lo' = 2^11 lo planes of P, Q and S (pass 2 of split_f16.h);
 //  * the unscale factors 2^-e(n), one float per column of the 32-column blocks;
-//  * one int per column of the 32-column blocks: bit 0 set when a piece of 8 consecutive k of
+//  * one int per column of the 32-column blocks: bit 0 set when a run of 4 consecutive k of
 //    P or Q of that column is nonzero and below the window (2^-3) at the column's scale, bit 1
 //    when the column is not flat (split_f16.h); the kernels' pass rules read them.
 __host__ __device__ inline int64_t complex_weight_split_vectors(int32_t Nc, int32_t Kc) {
@@ -683,9 +683,9 @@ static int complex_launch(const float* A_r, const float* A_i, int64_t lda, const
 
 // The unscale factor 2^-e(n) of every column of the 32-column blocks (1 past Nc): e(n) is the
 // exact scale (split_f16.h) of the column's largest magnitude over P, Q and P + Q.  flag[n]
-// bit 0 marks a column with a piece (8 consecutive k from a multiple of 8, as the fragments
-// hold them) of P or Q that is nonzero and below 2^-3 at that scale, bit 1 a column that is not
-// flat (a piece maximum, zero pieces included, below 2^-6 of the largest).
+// bit 0 marks a column with a run (4 consecutive k from a multiple of 4) of P or Q that is nonzero and
+// below 2^-3 at that scale, bit 1 a column that is not flat (the maximum of a piece of 8, zero pieces
+// included, below 2^-6 of the largest).
 __global__ void complex_weight_scale_kernel(const float* __restrict__ P, const float* __restrict__ Q, int64_t ldw,
                                             int32_t Nc, int32_t Kc, float* __restrict__ cinv, int* __restrict__ flag) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
@@ -703,11 +703,16 @@ __global__ void complex_weight_scale_kernel(const float* __restrict__ P, const f
   if (n < Nc)
     for (int k0 = 0; k0 < Kc; k0 += 8) {
       float mp = 0.0f, mq = 0.0f;
-      for (int k = k0; k < k0 + 8 && k < Kc; ++k) {
-        mp = fmaxf(mp, fabsf(P[(int64_t)n * ldw + k]));
-        mq = fmaxf(mq, fabsf(Q[(int64_t)n * ldw + k]));
+      for (int k1 = k0; k1 < k0 + 8 && k1 < Kc; k1 += 4) {
+        float rp = 0.0f, rq = 0.0f;
+        for (int k = k1; k < k1 + 4 && k < Kc; ++k) {
+          rp = fmaxf(rp, fabsf(P[(int64_t)n * ldw + k]));
+          rq = fmaxf(rq, fabsf(Q[(int64_t)n * ldw + k]));
+        }
+        low = low || f16_lossy(rp * pow2i(e)) || f16_lossy(rq * pow2i(e));
+        mp = fmaxf(mp, rp);
+        mq = fmaxf(mq, rq);
       }
-      low = low || f16_lossy(mp * pow2i(e)) || f16_lossy(mq * pow2i(e));
       pmin = fminf(pmin, fminf(mp, mq));
       pmax = fmaxf(pmax, fmaxf(mp, mq));
     }

@@ -44,8 +44,12 @@ __global__ void resident_weight_scale_kernel(const float* __restrict__ W, int64_
   if (n < N)
     for (int k0 = 0; k0 < K; k0 += 8) {
       float mp = 0.0f;
-      for (int k = k0; k < k0 + 8; ++k) mp = fmaxf(mp, fabsf(W[(int64_t)n * ldw + k]));
-      low = low || f16_lossy(mp * pow2i(e));
+      for (int k1 = k0; k1 < k0 + 8; k1 += 4) {
+        float mr = 0.0f;
+        for (int k = k1; k < k1 + 4; ++k) mr = fmaxf(mr, fabsf(W[(int64_t)n * ldw + k]));
+        low = low || f16_lossy(mr * pow2i(e));
+        mp = fmaxf(mp, mr);
+      }
       pmin = fminf(pmin, mp);
       pmax = fmaxf(pmax, mp);
     }

@@ -13,8 +13,10 @@
 //    registers, the next segment's in flight.  At most 168 VGPRs: three workgroups per CU;
 //  * a row's power-of-two scale is the exact one of its first nonzero segment, with one bit of
 //    headroom, lowered (and the accumulators with it) when a later segment would overflow: no pass
-//    over the row beforehand.  The window rule of split_f16.h is applied per segment against the
-//    weight's precomputed flags; a segment that fails it runs the products of pass 2;
+//    over the row beforehand.  The window rule of split_f16.h is applied per segment, to runs of 4
+//    elements, against the weight's precomputed flags; a segment that fails it runs the products of
+//    pass 2.  Small runs elsewhere in the row do not reach a segment's verdict, so a weight's own runs
+//    below the window always do (bit 0 of its flags);
 //  * the four partial tiles are summed once, in LDS, in wave order (bitwise reproducible), and the
 //    epilogues are those of the tiled kernels;
 //  * the column tiles of a row tile go to one XCD (its L2 then reads those rows of A once).
@@ -173,9 +175,6 @@ __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_til
       R = fmaxf(R, m[s]);
     }
     const float fac = sc.update(R), f = pow2i(sc.e);
-    bool low = false;
-#pragma unroll
-    for (int s = 0; s < S; ++s) low = low || f16_lossy(m[s] * f);
     if (__any(fac != 1.0f)) {
       float rs[16];
       row_factors(fac, fh, rs);
@@ -187,7 +186,15 @@ __device__ __forceinline__ void real_part(const Prob& p, int64_t row0, int n_til
     // The window rule of split_f16.h (a weight with a piece below its window always takes pass 2).
     // Pass 2: the residual planes hold 2^11 times the residuals, whose products are added to
     // accumulators scaled up by as much (exact), and scaled down again before hi * hi.
-    const bool two = (wbits & 1) || ((wbits & 2) && __any(low));
+    bool two = (wbits & 1) != 0;
+    if (wbits & 2) {
+      bool low = false;
+#pragma unroll
+      for (int s = 0; s < S; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) low = low || f16_lossy(amax4(raw[s][h]) * f);
+      two = two || __any(low);
+    }
     if (two) {
 #pragma unroll
       for (int j = 0; j < NB; ++j) {

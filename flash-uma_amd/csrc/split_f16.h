@@ -12,7 +12,8 @@
 // size 2^-22.  The accumulated output is multiplied by 2^-ea and 2^-eb afterwards (exact).
 //
 // Window.  The kernels stage a row in pieces (8 consecutive k of a row in the real GEMM, 4 of
-// each of a_r and a_i in the complex layer).  A piece is inside the window at a scale when its
+// each of a_r and a_i in the complex layer, 4 in the few-row kernels, whose scale is a segment's; a
+// pre-split weight is looked at in runs of 4).  A piece is inside the window at a scale when its
 // largest scaled magnitude is at or above 2^-3 (or it is zero) and no piece overflowed (largest
 // fp16 65504).  Inside it every element keeps 22 bits relative to the largest element of its
 // piece: |error(x)| <= 2^-22 max(|x|, max |piece|) 2^-e.  A piece below the window has the
@@ -164,9 +165,9 @@ constexpr int F16_PREPASS_CHUNKS = 4;
 //  * fp16 planes in MFMA-fragment order: per (32-column block, 16-k chunk), 3 x 64 lanes x 16 B:
 //    hi, lo and lo' = 2^11 lo of the column scaled by its exact power of two 2^e(n);
 //  * the unscale factors 2^-e(n), one float per column of the 32-column blocks;
-//  * one int per column of the 32-column blocks: bit 0 set when a piece (8 consecutive k from a
-//    multiple of 8) of the column is nonzero and below the window at the column's scale, bit 1
-//    when the column is not flat;
+//  * one int per column of the 32-column blocks: bit 0 set when a run (4 consecutive k from a
+//    multiple of 4) of the column is nonzero and below the window at the column's scale, bit 1
+//    when the column is not flat (pieces of 8);
 //  * one int (padded to 16 bytes): the OR of the column flags.
 __host__ __device__ inline int64_t resident_frag_vectors(int32_t N, int32_t K) {
   return (int64_t)((N + 31) / 32) * (K / 16) * 3 * 64;

@@ -325,7 +325,7 @@ int fu_complex_linear(const float* A_r, const float* A_i, int64_t lda, const flo
  * each column n scaled by a power of two 2^e(n) ([block][chunk][P hi, P lo, Q hi, Q lo, S hi,
  * S lo, P lo', Q lo', S lo'][64 lanes], lo' = 2^11 lo for the two-loop pass of the fp16 mode),
  * then the factors 2^-e(n) (one float per padded column), then one int32 per padded column:
- * bit 0 when 8 consecutive k of P or Q in that column are below the fp16 window at its scale,
+ * bit 0 when 4 consecutive k of P or Q in that column are below the fp16 window at its scale,
  * bit 1 when the column is not flat (a piece of 8 k more than 2^6 below its largest; the fp16
  * mode's pass rules read both): fu_complex_weight_split_bytes(Nc, Kc) bytes, 16-byte
  * aligned, valid in every matrix-core mode.  The bytes query returns a negative FU_ERR_* for Nc
@@ -340,7 +340,7 @@ int fu_complex_weight_split(const float* P, const float* Q, int64_t ldw, int32_t
  * (fu_linear_resident: K <= 128).  W2 receives the fp16 splits of every column n scaled by its
  * exact power of two 2^e(n) in MFMA-fragment order ([32-column block][16-k chunk][hi, lo, lo'
  * = 2^11 lo][64 lanes] x 16 bytes, zero padded to N = 32 n), then the factors 2^-e(n) (one float
- * per padded column), then one int32 per padded column (bit 0: 8 consecutive k below the fp16
+ * per padded column), then one int32 per padded column (bit 0: 4 consecutive k below the fp16
  * window at the column's scale; bit 1: the column is not flat), then their OR (one int32,
  * padded to 16 bytes): fu_linear_weight_split_bytes(N, K) bytes, 16-byte aligned.  The bytes
  * query returns a negative FU_ERR_* for a shape outside those bounds. */

@@ -138,6 +138,27 @@ def test_linear_short(cuda, M, N, K, ramp):
     assert (buf[:, N:] == 7.0).all() and e <= 1e-6 and e <= 1.5 * t + 1e-7, (e, t)
 
 
+@pytest.mark.parametrize("K", [64, 96, 640])
+@pytest.mark.parametrize("spread", [8, 12, 14])
+@pytest.mark.parametrize("seed", range(6))
+def test_linear_short_runs_of_four(cuda, K, spread, seed):
+    """Operands whose magnitude changes every 4 columns by powers of two up to 2^+-spread, against weights with
+    the inverse: a run of the weight below the window next to larger ones in its piece of 8 meets the
+    largest operands.  Every row at the tiled kernel's error and at the fp32 instructions'."""
+    from ops import _lib, linear
+    g = torch.Generator().manual_seed(100 * seed + K)
+    t = torch.randint(-spread, spread + 1, (K // 4,), generator=g).repeat_interleave(4)
+    x, W = torch.randn(65, K, generator=g) * torch.exp2(t), torch.randn(64, K, generator=g) / torch.exp2(t)
+    ref, x, W = x.double() @ W.double().T, x.to(cuda), W.to(cuda)
+    W2, y = linear.linear_weight_split(W), torch.empty(65, 64, device=cuda)
+    _lib.call("fu_linear_short", x.data_ptr(), K, W2.data_ptr(), None, y.data_ptr(), 64, 65, 64, K, _lib.stream_ptr(cuda))
+    with _lib.matmul_mode(_lib.MATMUL_FP32):
+        fp32 = linear.gemm(x, W)
+    e, f = (((v.double().cpu() - ref).norm(dim=1) / ref.norm(dim=1)).max().item() for v in (y, fp32))
+    # 22-bit operands down to 2^-27 of the largest, in fp32 sums: as the window cases of the tiled kernels
+    assert e <= 1.5 * f + 2e-7, (e, f)
+
+
 @pytest.mark.parametrize("M,K", [(49152, 320), (49153, 320)])
 def test_few_row_product_on_both_sides_of_its_line(cuda, monkeypatch, M, K):
     """gemm_few_rows at its last row count and past it: the two entry points, each at the bar above."""
