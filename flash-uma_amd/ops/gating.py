@@ -186,24 +186,14 @@ def _splits12(splits):
     return sp + (None,) * (12 - len(sp))
 
 
-# A block's convolution pair runs in the few-row kernels (csrc/gemm_short.hip, three launches each way) up
-# to SHORT_PAIR_MAX_EDGES edges and while its forward products stay below a number of operations.
-# Their time follows the operations; that of the tiled kernels, few workgroups walking K, hardly
-# depends on the edges and grows with the length of K, (lmax + 1) C, so the line lies higher for longer K.
-# Measured, us forward + backward, few-row captured | eager, tiled captured | eager (eager orders overlap on
-# a second stream), at the line's two sides in 1e10 operations:
-#   C  lmax   below: edges, few, tiled                      above
-#   64   2    0.90e10  13,107   220 | 209   249 | 331       1.47e10  21,299  341 | 321   299 | 325
-#   64   3    1.76e10  11,367   349 | 338   344 | 338       2.20e10  14,209  437 | 419   347 | 354
-#   64   4    1.76e10   6,318   328 | 307   342 | 328       2.20e10   7,898  406 | 388   373 | 337
-#   128  2    1.98e10   7,193   350 | 335   356 | 334       2.20e10   7,992  381 | 369   367 | 332
-#   128  3    2.20e10   3,552   370 | 344   447 | 355       2.53e10   4,085  416 | 394   446 | 369
-#   128  4    2.20e10   1,974   372 | 362   552 | 412       2.86e10   2,567  486 | 471   564 | 441
-#   256  2    2.20e10   1,998   361 | 352   533 | 400       2.86e10   2,597  478 | 478   540 | 426
-#   256  4    2.20e10     493   442 | 440  1040 | 710       2.86e10     641  616 | 614  1017 | 704
-SHORT_PAIR_MAX_EDGES = 16384
+# A block's convolution pair runs in the few-row kernels (csrc/gemm_short.hip, three launches each
+# way) up to this many floating-point operations in its forward products, and up to this many
+# edges; above either the tiled GEMMs fill the chip.  Measured, us forward + backward (captured,
+# few-row / tiled): C = 128 lmax 2 (2.75 MFLOP an edge) 282 / 354 at 6,000 edges, 549 / 459 at
+# 12,000; C = 128 lmax 4 (11.1) 327 / 554 at 1,620, 543 / 555 at 3,000; C = 64 lmax 2 (0.69) 194 /
+# 255 at 12,000, 303 / 291 at 20,000.
 SHORT_PAIR_MAX_FLOPS = 2.2e10
-SHORT_PAIR_BASE_FLOPS, SHORT_PAIR_FLOPS_PER_K = 1.3e10, 1.8e7
+SHORT_PAIR_MAX_EDGES = 16384
 
 
 @functools.lru_cache(maxsize=64)
@@ -225,8 +215,7 @@ def _short_pair(E: int, pair: tuple, sp: tuple, arrays, weights, *biases) -> boo
     pair's own shapes (another number of input or output channels, wider arrays and an unaligned conv2
     bias are the tiled kernels')."""
     flops, (w0, w1, w2), shapes = pair
-    most = min(SHORT_PAIR_MAX_FLOPS, SHORT_PAIR_BASE_FLOPS + SHORT_PAIR_FLOPS_PER_K * shapes[3][0])
-    return (0 < E <= SHORT_PAIR_MAX_EDGES and 0 < E * flops <= most
+    return (0 < E <= SHORT_PAIR_MAX_EDGES and 0 < E * flops <= SHORT_PAIR_MAX_FLOPS
             and tuple([x.shape for x in arrays]) == ((E, w0), (E, w1), (E, w2))
             and tuple([W.shape for W in weights]) == shapes and all([t is not None for t in sp])
             and all([b is not None and b.data_ptr() % 16 == 0 for b in biases])

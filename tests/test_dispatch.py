@@ -109,18 +109,3 @@ def test_few_row_product_dispatch(calls):
     assert calls[2:] == ["fu_linear"] * 2
     with pytest.raises(_lib.FlashUMAError):
         linear.gemm_few_rows(z(7, 256), W, W2, out)
-
-
-@pytest.mark.parametrize("C,L,E,few", [
-    (64, 2, 13107, True), (64, 2, 16384, True), (64, 2, 16385, False), (64, 3, 11000, True), (64, 3, 12788, False),
-    (64, 4, 6318, True), (64, 4, 7898, False), (128, 2, 7193, True), (128, 2, 7992, False), (128, 3, 3552, True),
-    (128, 3, 4085, False), (128, 4, 1974, True), (128, 4, 2567, False), (256, 2, 1998, True), (256, 2, 2597, False),
-    (256, 4, 493, True), (256, 4, 641, False)])
-def test_pair_goes_to_the_faster_kernels(calls, C, L, E, few):
-    """Both sides of the line between the few-row and the tiled pair, at edge counts where both were timed
-    (the figures stand at the rule)."""
-    from ops import gating
-    e = lambda *s: torch.empty(*s, device="meta")
-    for pair in gating._pair_shapes(C, L):
-        arrays, weights = [e(E, w) for w in pair[1]], [e(*s) for s in pair[2]]
-        assert gating._short_pair(E, pair, (0,) * 12, arrays, weights) is few
