@@ -186,12 +186,20 @@ def _splits12(splits):
     return sp + (None,) * (12 - len(sp))
 
 
-# A block's convolution pair runs in the few-row kernels (csrc/gemm_short.hip, three launches each
-# way) up to this many floating-point operations in its forward products, and up to this many
-# edges; above either the tiled GEMMs fill the chip.  Measured, us forward + backward (captured,
-# few-row / tiled): C = 128 lmax 2 (2.75 MFLOP an edge) 282 / 354 at 6,000 edges, 549 / 459 at
-# 12,000; C = 128 lmax 4 (11.1) 327 / 554 at 1,620, 543 / 555 at 3,000; C = 64 lmax 2 (0.69) 194 /
-# 255 at 12,000, 303 / 291 at 20,000.
+# A block's convolution pair runs in the few-row kernels (csrc/gemm_short.hip, three launches each way)
+# up to this many floating-point operations in its forward products, and up to this many edges; above
+# either the tiled GEMMs fill the chip.  The line is that of whole calls, us with the few-row / tiled pair just
+# below it (four layers; one layer for the block):
+#   C  lmax   edges     replayed step   eager step      embeddings      one block, eager
+#   64   3    14,040    3,275 / 3,193   4,046 / 5,149   1,720 / 2,186     856 / 1,163
+#   64   4     7,800    3,389 / 3,542   3,986 / 5,027   1,694 / 2,137     896 /   946
+#   128  2     7,890    2,707 / 2,833   3,440 / 4,702   1,268 / 1,816     814 / 1,106
+#   128  3     3,510    2,728 / 3,321   3,125 / 4,415   1,287 / 1,831     842 / 1,218
+# (eager, the tiled pair's calls cost more of the host's time).  The pair alone, captured, on random operands,
+# turns a little earlier where K is short (C = 64, lmax 3: 349 / 344 at 11,367 edges, 437 / 347 at 14,209;
+# C = 128, lmax 2: 350 / 356 at 7,193, 381 / 367 at 7,992) and later elsewhere (C = 128, lmax 4: 372 / 552 at
+# 1,974, 486 / 564 at 2,567; C = 256, lmax 2: 361 / 533 at 1,998, lmax 4: 442 / 1,040 at 493); C = 64, lmax 2
+# 220 / 249 at 13,107 edges, 271 / 261 at 16,384, 341 / 299 at 21,299.
 SHORT_PAIR_MAX_FLOPS = 2.2e10
 SHORT_PAIR_MAX_EDGES = 16384
 

@@ -109,3 +109,15 @@ def test_few_row_product_dispatch(calls):
     assert calls[2:] == ["fu_linear"] * 2
     with pytest.raises(_lib.FlashUMAError):
         linear.gemm_few_rows(z(7, 256), W, W2, out)
+
+
+@pytest.mark.parametrize("C,L,most", [(64, 2, 16384), (64, 3, 14209), (64, 4, 7898), (128, 2, 7992), (128, 4, 1974),
+                                      (256, 2, 1998), (256, 4, 493)])
+def test_pair_on_both_sides_of_its_line(calls, C, L, most):
+    """The last edge count of the few-row kernels and the first of the tiled ones, forward and backward."""
+    from ops import gating
+    e = lambda *s: torch.empty(*s, device="meta")
+    for pair in gating._pair_shapes(C, L):
+        for E in (1, most, most + 1):
+            arrays, weights = [e(E, w) for w in pair[1]], [e(*s) for s in pair[2]]
+            assert gating._short_pair(E, pair, (0,) * 12, arrays, weights) is (E <= most)
